@@ -171,6 +171,15 @@ int mbq_dequant_raw(int t, const uint8_t* raw_dev, int64_t rows, int64_t cols, f
 int mbq_matmul_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M, int64_t N, int64_t K, void* y_dev,
                    int out_dtype, void* stream);
 
+/* The same product for any number of activation rows (M >= 1), on the bfloat16 matrix cores with float32 accumulation:
+ * each weight value, bit for bit mbq_dequant_raw's, is cut into one to three bfloat16 terms whose sum it is exactly, so
+ * every product is exact as the float32 product of a bfloat16 x is up to its own rounding. Types, shapes and alignments
+ * as mbq_matmul_raw. work_dev: at least mbq_gemm_raw_work(M, N, K) bytes of device memory (16-byte aligned; NULL when
+ * that is 0) for the float32 partials of the K ranges, free again when the call's work on the stream is done. */
+int mbq_gemm_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M, int64_t N, int64_t K, void* y_dev,
+                 int out_dtype, void* work_dev, int64_t work_bytes, void* stream);
+int64_t mbq_gemm_raw_work(int64_t M, int64_t N, int64_t K);
+
 /* int8 per-output-channel linear: y (M, N) = (x (M, K) @ bf16(q).T accumulated in float32) * s, then out_dtype.
  * q_dev int8 (N, K) row-major, s_dev float32 (N,). Replaces linear(x, {"q", "s"}) (reference
  * src/mashbox/models/qwen3_8_27b/model.py:72-82); with out_dtype MBQ_OUT_F32 it returns the float32 y*s that the

@@ -276,24 +276,52 @@ int mbq_dequant_raw(int t, const uint8_t* raw_dev, int64_t rows, int64_t cols, f
     return launch_dequant_raw(t, raw_dev, rows, cols, w_dev, reinterpret_cast<hipStream_t>(stream));
 }
 
+// checks shared by the products on the file's blocks
+static int raw_product_args(const char* what, int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M, int64_t N, int64_t K,
+                            void* y_dev) {
+    if (N <= 0 || K <= 0 || N > INT32_MAX || K > INT32_MAX || M * K > INT32_MAX || M * N > INT32_MAX)
+        return set_error(MBQ_BAD_ARG, "%s: shape (%lld, %lld, %lld)", what, (long long)M, (long long)N, (long long)K);
+    if (K % 32 || K % ggml_block(t).values)
+        return set_error(MBQ_BAD_ARG, "%s: K = %lld must be a multiple of 32 and of the block size %d", what, (long long)K,
+                         ggml_block(t).values);
+    if (!raw_dev || !x_dev || !y_dev || !aligned16(x_dev) || (reinterpret_cast<uintptr_t>(y_dev) & 3u))
+        return set_error(MBQ_BAD_ARG, "%s: raw, x or y is NULL, x not 16-byte or y not 4-byte aligned", what);
+    if (reinterpret_cast<uintptr_t>(raw_dev) % raw_block_align(t))
+        return set_error(MBQ_BAD_ARG, "%s: the blocks must start at a multiple of %d bytes", what, raw_block_align(t));
+    return 0;
+}
+
 int mbq_matmul_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M, int64_t N, int64_t K, void* y_dev,
                    int out_dtype, void* stream) {
     if (!raw_type(t) || is_type(t))
         return set_error(MBQ_BAD_ARG, "matmul_raw takes the file blocks of an exact-path type without kernel planes, not type %d", t);
-    if (out_dtype != MBQ_OUT_F32 && out_dtype != MBQ_OUT_BF16) return set_error(MBQ_BAD_ARG, "out_dtype %d", out_dtype);
+    if (int rc = check_out(out_dtype)) return rc;
     if (M == 0) return MBQ_OK;
     if (M < 0 || M > 8)
-        return set_error(MBQ_BAD_ARG, "matmul_raw: M = %lld (1-8 rows; more rows: mbq_dequant_raw and a GEMM)", (long long)M);
-    if (N <= 0 || K <= 0 || N > INT32_MAX || K > INT32_MAX || M * K > INT32_MAX || M * N > INT32_MAX)
-        return set_error(MBQ_BAD_ARG, "matmul_raw: shape (%lld, %lld, %lld)", (long long)M, (long long)N, (long long)K);
-    if (K % 32 || K % ggml_block(t).values)
-        return set_error(MBQ_BAD_ARG, "matmul_raw: K = %lld must be a multiple of 32 and of the block size %d", (long long)K,
-                         ggml_block(t).values);
-    if (!raw_dev || !x_dev || !y_dev || !aligned16(x_dev) || (reinterpret_cast<uintptr_t>(y_dev) & 3u))
-        return set_error(MBQ_BAD_ARG, "matmul_raw: raw, x or y is NULL, x not 16-byte or y not 4-byte aligned");
-    if (reinterpret_cast<uintptr_t>(raw_dev) % raw_block_align(t))
-        return set_error(MBQ_BAD_ARG, "matmul_raw: the blocks must start at a multiple of %d bytes", raw_block_align(t));
+        return set_error(MBQ_BAD_ARG, "matmul_raw: M = %lld (1-8 rows; more rows: mbq_gemm_raw)", (long long)M);
+    if (int rc = raw_product_args("matmul_raw", t, raw_dev, x_dev, M, N, K, y_dev)) return rc;
     return launch_raw_gemv(t, raw_dev, x_dev, M, N, K, y_dev, out_dtype == MBQ_OUT_BF16 ? 1 : 0,
+                           reinterpret_cast<hipStream_t>(stream));
+}
+
+int64_t mbq_gemm_raw_work(int64_t M, int64_t N, int64_t K) {
+    if (M < 0 || N <= 0 || K <= 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX)
+        return set_error(MBQ_BAD_ARG, "gemm_raw: shape (%lld, %lld, %lld)", (long long)M, (long long)N, (long long)K);
+    return M == 0 ? 0 : raw_gemm_work(M, N, K);
+}
+
+int mbq_gemm_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M, int64_t N, int64_t K, void* y_dev,
+                 int out_dtype, void* work_dev, int64_t work_bytes, void* stream) {
+    if (!raw_type(t) || is_type(t))
+        return set_error(MBQ_BAD_ARG, "gemm_raw takes the file blocks of an exact-path type without kernel planes, not type %d", t);
+    if (int rc = check_out(out_dtype)) return rc;
+    if (M == 0) return MBQ_OK;
+    if (M < 0 || M > INT32_MAX) return set_error(MBQ_BAD_ARG, "gemm_raw: M = %lld", (long long)M);
+    if (int rc = raw_product_args("gemm_raw", t, raw_dev, x_dev, M, N, K, y_dev)) return rc;
+    const int64_t need = raw_gemm_work(M, N, K);
+    if (work_bytes < need || (need > 0 && (!work_dev || !aligned16(work_dev))))
+        return set_error(MBQ_BAD_ARG, "gemm_raw: %lld bytes of work needed (16-byte aligned), %lld given", (long long)need, (long long)work_bytes);
+    return launch_raw_gemm(t, raw_dev, x_dev, M, N, K, y_dev, out_dtype == MBQ_OUT_BF16 ? 1 : 0, static_cast<float*>(work_dev),
                            reinterpret_cast<hipStream_t>(stream));
 }
 

@@ -1,0 +1,408 @@
+// gfx950 kernels of the exact path's fused products: y (M, N) = x (M, K) @ W.T straight from the file's blocks of the
+// ggml types without kernel planes, each weight value rebuilt in registers (mbq_raw_unit.h: bit for bit the values
+// mbq_dequant_raw writes) instead of written as float32 and read back. Reference src/mashbox/ops/__init__.py:574-576,
+// 624-632 (dequant, then a float32 dot).
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+
+#include "mbq_device.h"
+#include "mbq_launch.h"
+#include "mbq_layout.h"
+#include "mbq_raw_unit.h"
+
+namespace mbq {
+
+static int check_launch(const char* what) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(MBQ_LAUNCH_FAIL, "%s: %s", what, hipGetErrorString(e));
+    return 0;
+}
+
+// ------------------------------------------------------------------------------------------------ 1-8 rows
+// The exact path's product for one to eight activation rows, fused: y (M, N) = x (M, K) @ W.T with W's rows rebuilt
+// from the file's blocks in registers (raw_unit, bit for bit the values mbq_dequant_raw writes), float32 products and
+// sums, each row read once from HBM instead of written as float32 and read back (reference src/mashbox/ops/__init__.py
+// :574-576, 624-632: dequant, then a float32 dot). Lanes in groups of LPR take one weight row each (4 waves x 64 / LPR
+// rows per block, rows over the grid), a lane the row's 32-value units u = lane % LPR, + LPR, ...; the group's sums
+// meet by shuffles; with U2 a lane has two units' loads in flight. Up to RGV_MAX_M activation rows, one float32 sum
+// each in registers.
+constexpr int RGV_MAX_M = 8;
+template <int T, int LPR, bool U2>
+__global__ __launch_bounds__(256) void raw_gemv_kernel(const uint8_t* __restrict__ raw, const uint16_t* __restrict__ x,
+                                                       int M, int N, int K, void* __restrict__ y, int out_bf16) {
+    constexpr int RPB = 256 / LPR;                                       // rows per block
+    const int lane = threadIdx.x & (LPR - 1);
+    const int U = K >> 5;
+    const int64_t rb = raw_row_bytes<T>(K);
+    for (int64_t n = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR; n < N; n += (int64_t)gridDim.x * RPB) {
+        float acc[RGV_MAX_M];
+#pragma unroll
+        for (int m = 0; m < RGV_MAX_M; ++m) acc[m] = 0.f;
+        const uint8_t* row = raw + n * rb;
+        for (int u0 = lane; u0 < U; u0 += (U2 ? 2 : 1) * LPR)
+#pragma unroll
+        for (int uu = 0; uu < (U2 ? 2 : 1); ++uu) {
+            const int u = u0 + uu * LPR;
+            if (u >= U) break;
+            float v[32];
+            raw_unit<T>(row, u, v);
+#pragma unroll
+            for (int m = 0; m < RGV_MAX_M; ++m) {
+                if (m < M) {
+                    const u32x4* xp = reinterpret_cast<const u32x4*>(x + (int64_t)m * K + 32 * u);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const u32x4 q = xp[c];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            acc[m] = __builtin_fmaf(__uint_as_float(q[e] << 16), v[8 * c + 2 * e], acc[m]);
+                            acc[m] = __builtin_fmaf(__uint_as_float(q[e] & 0xFFFF0000u), v[8 * c + 2 * e + 1], acc[m]);
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < RGV_MAX_M; ++m)
+#pragma unroll
+            for (int off = LPR / 2; off >= 1; off >>= 1) acc[m] += __shfl_xor(acc[m], off, LPR);
+        if (lane == 0) {
+#pragma unroll
+            for (int m = 0; m < RGV_MAX_M; ++m) {
+                if (m < M) {
+                    if (out_bf16) reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)bf16_bits(acc[m]);
+                    else reinterpret_cast<float*>(y)[(int64_t)m * N + n] = acc[m];
+                }
+            }
+        }
+    }
+}
+
+// Lanes per row by the row's 32-value units U (MI355X, interleaved timings of 16, 32 and 64 lanes, with and without two
+// units in flight, on Q2_K 9728 x 2560, Q3_K 17408 x 5120, IQ4_XS 5120 x 17408, Q5_0 6144 x 5120 at 4 rows and F16
+// 4096 x 4096): short rows (U < 128) 16 lanes, so that a wave holds 4 rows (Q2_K 14.5 -> 10.8 us); the 256-value types,
+// whose units cost the most vector work, 32 lanes up to U = 256 (Q3_K 51.3 -> 46.5 us); else 64, with two units in
+// flight from U = 256 on (IQ4_XS 66.1 -> 60.8 us). Each choice was the fastest or within 2 % of it on those cases.
+template <int T>
+static void raw_gemv_t(const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16,
+                       hipStream_t s) {
+    const int64_t U = K / 32;
+    constexpr bool HEAVY = ggml_block(T).values == 256;
+    if (U < 128)
+        raw_gemv_kernel<T, 16, false><<<dim3((unsigned)((N + 15) / 16)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
+    else if (HEAVY && U < 256)
+        raw_gemv_kernel<T, 32, false><<<dim3((unsigned)((N + 7) / 8)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
+    else if (U < 256)
+        raw_gemv_kernel<T, 64, false><<<dim3((unsigned)((N + 3) / 4)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
+    else
+        raw_gemv_kernel<T, 64, true><<<dim3((unsigned)((N + 3) / 4)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
+}
+
+int launch_raw_gemv(int t, const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16,
+                    hipStream_t s) {
+    switch (t) {
+        case T_F32: raw_gemv_t<T_F32>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_F16: raw_gemv_t<T_F16>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_BF16: raw_gemv_t<T_BF16>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_Q4_1: raw_gemv_t<T_Q4_1>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_Q5_0: raw_gemv_t<T_Q5_0>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_Q5_1: raw_gemv_t<T_Q5_1>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_Q2_K: raw_gemv_t<T_Q2_K>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_Q3_K: raw_gemv_t<T_Q3_K>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_IQ4_NL: raw_gemv_t<T_IQ4_NL>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_IQ4_XS: raw_gemv_t<T_IQ4_XS>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_TQ1_0: raw_gemv_t<T_TQ1_0>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_TQ2_0: raw_gemv_t<T_TQ2_0>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_MXFP4: raw_gemv_t<T_MXFP4>(raw, x, M, N, K, y, out_bf16, s); break;
+        case T_NVFP4: raw_gemv_t<T_NVFP4>(raw, x, M, N, K, y, out_bf16, s); break;
+        default: return set_error(MBQ_BAD_ARG, "raw GEMV: no kernel for ggml type %d (kernel types run on their planes)", t);
+    }
+    return check_launch("raw GEMV");
+}
+
+
+// ------------------------------------------------------------------------------------- more rows: a bfloat16-split GEMM
+// The float32 product on the bfloat16 matrix cores. x is bfloat16 as it comes; every weight value is the exact sum of
+// raw_terms<T>() bfloat16 terms (its float32 bits cut into 8-bit significands: the top, then what is left, then the
+// rest), so the MFMAs multiply exactly and only their float32 accumulation rounds, as a float32 GEMM's does. Against a
+// float64 product (2-norm, 512 x 4096 x 5120) it is off by 1.5e-7 to 2.7e-7, the rebuild and float32 library GEMM it
+// replaces by 0.7e-6 to 1.3e-6; smaller shapes alike. The float32 GEMM runs at 98 TFLOP/s here; this kernel's MFMAs at
+// 1.25 PFLOP/s, 418 TFLOP/s of the product with three terms, 582 with two, 749 with one (512 rows, 34816 x 5120: IQ4_XS
+// 436 us, Q5_0 313, BF16 244; the rebuild and float32 GEMM 2.2 ms).
+//
+// Tile: 32 BMT activation rows x 256 weight rows, K step 64, 8 waves. Wave w owns weight rows 32w .. 32w + 31 and all
+// the activation rows (BMT accumulators of v_mfma_f32_32x32x16_bf16): its lane l decodes unit l / 32 of the K step of row
+// l % 32 straight into B operands, so no weight passes LDS and no value is decoded twice in a block; x goes through an
+// LDS ring of three stages filled by DMA two steps ahead. The K values of an MFMA are the 8 of each lane half's unit
+// (values 8s .. 8s + 7 of units 0 and 1 at substep s), for A and B alike. Bound: the matrix cores (BMT = 8: 96 MFMAs of
+// 32 cycles per wave and step, against about 300 vector instructions of decode and split).
+//
+// One barrier per step. The weight bytes of the next step and the x stage after it are issued after it, weights first,
+// so that at the next barrier's wait only that DMA may be outstanding: the wait counts DMA instructions alone.
+//
+// The tiles that do not fill a round of the CUs are cut along K into S pieces, each a block of its own, whose float32
+// partials the second kernel adds in piece order. Where an output comes out NaN (a non-finite weight or activation,
+// whose lower terms are inf - inf or meet 0 * inf), it is recomputed value by value, so that it is what the float32
+// product gives.
+constexpr int RG_T = 512, RG_BN = 256, RG_K = 64;
+
+struct RawGemmArgs {
+    const uint8_t* raw;
+    const uint16_t* x;
+    void* y;
+    float* part;
+    int M, N, K, out_bf16;
+    int tm;                // tiles along M (fastest)
+    int full, S, ipp;      // tiles run whole; pieces per other tile, K steps per piece
+};
+
+// one output in float32, value by value
+template <int T>
+__device__ __forceinline__ float raw_dot(const uint8_t* row, const uint16_t* x, int K) {
+    float acc = 0.f;
+    for (int u = 0; u < K / 32; ++u) {
+        RawRegs<T> r;
+        raw_load<T>(r, row, u);
+        const RawScales sc = raw_scales<T>(r, u);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            float v[8];
+            raw_vals<T>(r, sc, u, s, v);
+            const u32x4 q = ld16(x + 32 * u + 8 * s);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                acc = __builtin_fmaf(__uint_as_float((e & 1) ? q[e >> 1] & 0xFFFF0000u : q[e >> 1] << 16), v[e], acc);
+        }
+    }
+    return acc;
+}
+
+// element offset of chunk c (8 values) of row r in an x stage
+__device__ __forceinline__ int rg_off(int r, int c) { return r * RG_K + ((c ^ ((r >> 1) & 7)) << 3); }
+
+// 8 values -> NT bfloat16 operands whose sum they are
+template <int NT>
+__device__ __forceinline__ void raw_split(const float v[8], bf16x8_t b[NT]) {
+#pragma clang fp contract(off)                                          // v's own bits: not the product behind them, unrounded
+    uint32_t t[NT][4];
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = v[e];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) t[k][e >> 1] = __builtin_amdgcn_perm(__float_as_uint(f[e + 1]), __float_as_uint(f[e]), 0x07060302u);
+        if (k + 1 < NT)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] -= __uint_as_float(__float_as_uint(f[e]) & 0xFFFF0000u);
+        b[k] = __builtin_bit_cast(bf16x8_t, u32x4{t[k][0], t[k][1], t[k][2], t[k][3]});
+    }
+}
+
+template <int T, int BMT>
+__global__ __launch_bounds__(RG_T, BMT >= 4 || T == T_TQ1_0 ? 2 : 4) void raw_gemm_kernel(const RawGemmArgs g) {
+    constexpr int NT = raw_terms<T>(), BM = 32 * BMT, STAGE = BM * RG_K;
+    constexpr int ND = BMT >= 2 ? BMT / 2 : 1;                           // DMA instructions of a wave per stage
+    extern __shared__ __align__(16) uint16_t lds[];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+    const int IT = (g.K + RG_K - 1) / RG_K, U = g.K >> 5;
+    const int b = blockIdx.x, p = b - g.full;
+    const int tile = p < 0 ? b : g.full + p / g.S;
+    const int k0 = p < 0 ? 0 : (p % g.S) * g.ipp, k1 = p < 0 ? IT : (k0 + g.ipp < IT ? k0 + g.ipp : IT);
+    const int m0 = (tile % g.tm) * BM, n = (tile / g.tm) * RG_BN + wave * 32 + col;
+    const uint8_t* row = g.raw + (int64_t)(n < g.N ? n : g.N - 1) * raw_row_bytes<T>(g.K);
+
+    // x DMA: instruction i of wave w fills stage rows 8 (w ND + i) .. + 7 (BMT = 1: waves 4-7 fill the rows of 0-3 again,
+    // with the same bytes); lane l the 16 bytes at l, whose chunk the row's swizzle names
+    const rsrc_t xr = make_rsrc(g.x + (int64_t)m0 * g.K, (uint32_t)((g.M - m0 < BM ? g.M - m0 : BM) * g.K * 2));
+    uint32_t vo[ND], vl[ND];
+    uint16_t* dst[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const int r0 = 8 * ((wave * ND + i) % (4 * BMT)), r = r0 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        vo[i] = m0 + r < g.M ? (uint32_t)(r * g.K + 8 * c) * 2u : OOB_VOFF;
+        vl[i] = 64 * (IT - 1) + 8 * c < g.K ? vo[i] : OOB_VOFF;          // the last step's chunks past K read zero
+        dst[i] = lds + r0 * RG_K;
+    }
+    // every step issues its weight loads and its DMA, past the end too (the last unit again; zeros into a stage that is not
+    // read): the compiler then knows, on every path, which loads a wait covers
+    auto dma = [&](int it, int stage) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+            dma16(xr, dst[i] + stage * STAGE, it >= k1 ? OOB_VOFF : it == IT - 1 ? vl[i] : vo[i], (uint32_t)it * (RG_K * 2));
+    };
+    // a K of an odd number of units: the second half's unit past K is its last unit again (it meets zeros)
+    auto unit = [&](int it) { const int u = 2 * (it < k1 ? it : k1 - 1) + half; return u < U ? u : U - 1; };
+
+    f32x16_t acc[BMT];
+#pragma unroll
+    for (int r = 0; r < BMT; ++r)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[r][i] = 0.f;
+    RawRegs<T> cur, nxt;
+    dma(k0, 0);
+    asm volatile("" ::: "memory");
+    raw_load<T>(cur, row, unit(k0));
+    asm volatile("" ::: "memory");
+    dma(k0 + 1, 1);
+
+    int st0 = 0, st2 = 2;                                                 // this step's stage; the one two steps on
+    for (int it = k0; it < k1; ++it) {
+        wait_vm<ND>();                                                    // all but the next stage's DMA has landed
+        wait_lgkm0();                                                     // and the last step's reads of the stage DMA fills next
+        barrier_nofence();
+        raw_load<T>(nxt, row, unit(it + 1));
+        asm volatile("" ::: "memory");
+        dma(it + 2, st2);
+        const int u = unit(it);
+        const RawScales sc = raw_scales<T>(cur, u);
+        const uint16_t* st = lds + st0 * STAGE;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            float v[8];
+            raw_vals<T>(cur, sc, u, s, v);
+            bf16x8_t bt[NT], a[BMT];
+            raw_split<NT>(v, bt);
+#pragma unroll
+            for (int r = 0; r < BMT; ++r) a[r] = __builtin_bit_cast(bf16x8_t, ld16(st + rg_off(32 * r + col, 4 * half + s)));
+#pragma unroll
+            for (int k = 0; k < NT; ++k)
+#pragma unroll
+                for (int r = 0; r < BMT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r], bt[k], acc[r], 0, 0, 0);
+        }
+        cur = nxt;
+        st0 = st0 == 2 ? 0 : st0 + 1;
+        st2 = st2 == 2 ? 0 : st2 + 1;
+    }
+    wait_vm<0>();                                                         // no DMA outlives the block's LDS
+
+    if (p >= 0) {                                                         // a piece: its partial tile
+        float* o = g.part + ((int64_t)p * BM + 4 * half) * RG_BN + wave * 32 + col;
+#pragma unroll
+        for (int r = 0; r < BMT; ++r)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[(32 * r + 8 * (i >> 2) + (i & 3)) * RG_BN] = acc[r][i];
+        return;
+    }
+    uint32_t bad[(BMT + 1) / 2] = {};                                     // the lane's NaN outputs, a bit each
+    auto store = [&](auto bf16) {
+#pragma unroll
+        for (int r = 0; r < BMT; ++r)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int m = m0 + 32 * r + 8 * (i >> 2) + 4 * half + (i & 3);
+                if (m < g.M && n < g.N) {
+                    store_y(g.y, (int64_t)m * g.N + n, acc[r][i], decltype(bf16)::value);
+                    bad[r >> 1] |= acc[r][i] != acc[r][i] ? 1u << (16 * (r & 1) + i) : 0u;
+                }
+            }
+    };
+    if (g.out_bf16) store(std::true_type{});
+    else store(std::false_type{});
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < (BMT + 1) / 2; ++i) any |= bad[i];
+    if (any == 0) return;
+    for (int j = 0; j < 16 * BMT; ++j) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int i = 0; i < (BMT + 1) / 2; ++i) w = (j >> 5) == i ? bad[i] : w;
+        if (!((w >> (j & 31)) & 1u)) continue;
+        const int m = m0 + 32 * (j >> 4) + 8 * ((j >> 2) & 3) + 4 * half + (j & 3);
+        store_y(g.y, (int64_t)m * g.N + n, raw_dot<T>(row, g.x + (int64_t)m * g.K, g.K), g.out_bf16);
+    }
+}
+
+// the cut tiles' outputs: the S partials of each added in piece order (4 columns a thread), then y
+template <int T>
+__global__ __launch_bounds__(256) void raw_reduce_kernel(const RawGemmArgs g, int BM) {
+    const int e = (int)(blockIdx.x * 256 + threadIdx.x) * 4, tile = g.full + blockIdx.y;
+    const int m = (tile % g.tm) * BM + e / RG_BN, n0 = (tile / g.tm) * RG_BN + e % RG_BN;
+    if (m >= g.M || n0 >= g.N) return;
+    const float* q = g.part + (int64_t)blockIdx.y * g.S * BM * RG_BN + e;
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(q);
+    for (int s = 1; s < g.S; ++s) v += *reinterpret_cast<const f32x4_t*>(q + (int64_t)s * BM * RG_BN);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = n0 + i;
+        if (n >= g.N) break;
+        float f = v[i];
+        if (f != f) f = raw_dot<T>(g.raw + (int64_t)n * raw_row_bytes<T>(g.K), g.x + (int64_t)m * g.K, g.K);
+        store_y(g.y, (int64_t)m * g.N + n, f, g.out_bf16);
+    }
+}
+
+// The plan of an (M, N, K) product: rows per tile, the tiles run whole and the cut of the rest.
+struct RawPlan { int bmt, tm, tiles, full, S, ipp; };
+static RawPlan raw_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    RawPlan p{};
+    p.bmt = M <= 32 ? 1 : M <= 64 ? 2 : M <= 128 ? 4 : 8;
+    p.tm = (int)((M + 32 * p.bmt - 1) / (32 * p.bmt));
+    const int64_t tiles = p.tm * ((N + RG_BN - 1) / RG_BN), IT = (K + RG_K - 1) / RG_K;
+    const int64_t P = (int64_t)cus;
+    int64_t rem = tiles % P, best = 0, bs = 1;
+    p.full = (int)(tiles - rem);
+    // the rest in S pieces: the fewest K steps of the busiest CU, a piece's partial counted as two steps
+    for (int64_t S = 1; rem > 0 && S <= 32 && S <= IT; ++S) {
+        const int64_t ipp = (IT + S - 1) / S, pieces = rem * ((IT + ipp - 1) / ipp);
+        const int64_t cost = (pieces + P - 1) / P * (ipp + (S > 1 ? 2 : 0)) + (S > 1 ? 4 : 0);
+        if (S == 1 || cost < best) best = cost, bs = S;
+    }
+    if (rem == 0 || bs == 1) {
+        p.full = (int)tiles;
+        p.S = 1;
+        p.ipp = (int)IT;
+    } else {
+        p.ipp = (int)((IT + bs - 1) / bs);
+        p.S = (int)((IT + p.ipp - 1) / p.ipp);
+    }
+    p.tiles = (int)tiles;
+    return p;
+}
+
+int64_t raw_gemm_work(int64_t M, int64_t N, int64_t K) {
+    const RawPlan p = raw_plan(M, N, K, cus_of_device());
+    return (int64_t)(p.tiles - p.full) * p.S * 32 * p.bmt * RG_BN * 4;
+}
+
+template <int T, int BMT>
+static int raw_gemm_b(const RawGemmArgs& g, const RawPlan& p, hipStream_t s) {
+    constexpr size_t lds = (size_t)3 * 32 * BMT * RG_K * 2;
+    auto kern = raw_gemm_kernel<T, BMT>;
+    static std::atomic<uint64_t> set{0};
+    if (set_lds_limit((const void*)kern, lds, set) != hipSuccess) return set_error(MBQ_LAUNCH_FAIL, "raw GEMM: %zu bytes of LDS refused", lds);
+    const int rem = p.tiles - p.full;
+    kern<<<dim3((unsigned)(p.full + rem * p.S)), RG_T, lds, s>>>(g);
+    if (rem > 0) raw_reduce_kernel<T><<<dim3((unsigned)(32 * BMT * RG_BN / 1024), (unsigned)rem), 256, 0, s>>>(g, 32 * BMT);
+    return check_launch("raw GEMM");
+}
+
+template <int T>
+static int raw_gemm_t(const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16, float* work,
+                      hipStream_t s) {
+    const RawPlan p = raw_plan(M, N, K, cus_of_device());
+    const RawGemmArgs g{raw, x, y, work, (int)M, (int)N, (int)K, out_bf16, p.tm, p.full, p.S, p.ipp};
+    switch (p.bmt) {
+        case 1: return raw_gemm_b<T, 1>(g, p, s);
+        case 2: return raw_gemm_b<T, 2>(g, p, s);
+        case 4: return raw_gemm_b<T, 4>(g, p, s);
+        default: return raw_gemm_b<T, 8>(g, p, s);
+    }
+}
+
+int launch_raw_gemm(int t, const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16,
+                    float* work, hipStream_t s) {
+    switch (t) {
+#define RAW_CASE(T) case T: return raw_gemm_t<T>(raw, x, M, N, K, y, out_bf16, work, s);
+        RAW_CASE(T_F32) RAW_CASE(T_F16) RAW_CASE(T_BF16) RAW_CASE(T_Q4_1) RAW_CASE(T_Q5_0) RAW_CASE(T_Q5_1) RAW_CASE(T_Q2_K)
+        RAW_CASE(T_Q3_K) RAW_CASE(T_IQ4_NL) RAW_CASE(T_IQ4_XS) RAW_CASE(T_TQ1_0) RAW_CASE(T_TQ2_0) RAW_CASE(T_MXFP4) RAW_CASE(T_NVFP4)
+#undef RAW_CASE
+    }
+    return set_error(MBQ_BAD_ARG, "raw GEMM: no kernel for ggml type %d (kernel types run on their planes)", t);
+}
+
+}  // namespace mbq

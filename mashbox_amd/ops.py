@@ -49,6 +49,7 @@ import sys
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -439,21 +440,40 @@ def _blocks(h: Raw) -> torch.Tensor:
 RAW_GEMV_MAX_M = 8                    # activation rows mbq_matmul_raw takes
 
 
-def _raw_gemv(x: torch.Tensor, h: "Raw") -> torch.Tensor | None:
-    """the fused exact-path product for a bfloat16 x of 1-8 rows on a type without kernel planes (mbq_matmul_raw: each
-    weight row rebuilt in registers and multiplied in float32, result rounded to bfloat16); None where it does not apply
-    (other dtypes: the reference multiplies float32 x, not its bfloat16 rounding)"""
+def _untraced(x: torch.Tensor) -> bool:
+    """x is an ordinary tensor outside every transform: no gradient is recorded for it (reverse or forward mode), no vmap
+    or other function transform runs and nothing traces. The exact path's torch operations serve those."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not (x.requires_grad and torch.is_grad_enabled())
+            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def _raw_product(x: torch.Tensor, h: "Raw") -> torch.Tensor | None:
+    """the fused exact-path product of a bfloat16 x on a type without kernel planes: each weight value rebuilt in registers
+    and multiplied exactly, float32 sums, result rounded to bfloat16 (1-8 rows: mbq_matmul_raw; more: mbq_gemm_raw). None
+    where it does not apply (other dtypes: the reference multiplies float32 x, not its bfloat16 rounding; sizes past the
+    kernels' 32-bit counts; more than 8 rows that something differentiates, transforms or traces)"""
     rows, cols = h.shape[-2:]
     lead = tuple(x.shape[:-1])
     m = int(np.prod(lead, dtype=np.int64)) if lead else 1
-    if (x.dtype != torch.bfloat16 or not 1 <= m <= RAW_GEMV_MAX_M or h.t in (2, 8, 12, 13, 14)
-            or cols % max(32, TYPES[h.t][1])):
+    if (x.dtype != torch.bfloat16 or m < 1 or h.t in (2, 8, 12, 13, 14) or cols % max(32, TYPES[h.t][1])
+            or (m > RAW_GEMV_MAX_M and (max(m * cols, m * rows) > 0x7FFFFFFF or not _untraced(x)))):
         return None                                  # (the kernel types' blocks, off the kernels: rebuild and GEMM)
     blocks = _blocks(h).reshape(rows, -1).contiguous()
     x2 = x.reshape(m, cols).to(blocks.device).contiguous()
     y = torch.empty((m, rows), dtype=torch.bfloat16, device=blocks.device)
-    _lib.check(_lib.lib().mbq_matmul_raw(int(h.t), ctypes.c_void_p(blocks.data_ptr()), ctypes.c_void_p(x2.data_ptr()), m,
-                                         rows, cols, ctypes.c_void_p(y.data_ptr()), 1, _stream()), "matmul_raw")
+    lib = _lib.lib()
+    p = ctypes.c_void_p
+    if m <= RAW_GEMV_MAX_M:
+        _lib.check(lib.mbq_matmul_raw(int(h.t), p(blocks.data_ptr()), p(x2.data_ptr()), m, rows, cols, p(y.data_ptr()), 1,
+                                      _stream()), "matmul_raw")
+    else:
+        if x2.data_ptr() % 16:                       # a view at an odd offset: the kernel copies 16 bytes at a time
+            x2 = x2.clone()
+        nwork = _lib.check(lib.mbq_gemm_raw_work(m, rows, cols), "gemm_raw_work")
+        work = torch.empty(nwork, dtype=torch.uint8, device=blocks.device)
+        _lib.check(lib.mbq_gemm_raw(int(h.t), p(blocks.data_ptr()), p(x2.data_ptr()), m, rows, cols, p(y.data_ptr()), 1,
+                                    p(work.data_ptr()), nwork, _stream()), "gemm_raw")
     return y.reshape(lead + (rows,))
 
 
@@ -520,7 +540,7 @@ def qmatmul(x: torch.Tensor, h) -> torch.Tensor:
     if isinstance(h, Raw):
         if h.raw.dim() > 2:
             raise ValueError(f"{h}: a stack is multiplied one layer at a time (index the stack)")
-        y = _raw_gemv(x, h)
+        y = _raw_product(x, h)
         return y if y is not None else _exact_matmul(x, h).to(x.dtype)
     raise TypeError(f"qmatmul: not a weight handle: {h!r}")
 
