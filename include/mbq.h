@@ -162,8 +162,10 @@ int mbq_dequant_raw(int t, const uint8_t* raw_dev, int64_t rows, int64_t cols, f
 
 /* y (M, N) = x (M, K) bf16 @ W.T for 1-8 activation rows, W (N, K) the file's blocks raw_dev (N, row_bytes) of a type
  * mbq_has_raw_type names that has no kernel planes (F32, F16, BF16, Q4_1, Q5_0, Q5_1, Q2_K, Q3_K, IQ4_NL, IQ4_XS,
- * TQ1_0, TQ2_0, MXFP4, NVFP4): each weight row rebuilt in registers, bit for bit the values of mbq_dequant_raw, and
- * multiplied in float32 (float32 products summed in float32), without writing W. K must be a multiple of 32; M = 0
+ * TQ1_0, TQ2_0, MXFP4, NVFP4), in float32 and without writing W: F32, F16 and TQ1_0 values rebuilt in registers, bit for
+ * bit mbq_dequant_raw's, float32 products and sums; of the other types the integer codes of 16 or 32 values multiplied
+ * exactly and summed in float32, the sum times their block scale (value by value where a scale, an
+ * activation or a sum is not finite). K must be a multiple of 32; M = 0
  * launches nothing; more than 8 rows is refused (mbq_dequant_raw and a GEMM serve those). The exact path's product of
  * reference src/mashbox/ops/__init__.py:574-576,624-632 (dequant, then a float32 dot) for decode-sized batches.
  * raw_dev starts at a multiple of the type's block alignment (4 bytes for Q2_K, Q4_1, Q5_1, IQ4_XS, NVFP4 and F32; 2

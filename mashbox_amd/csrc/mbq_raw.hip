@@ -23,107 +23,184 @@ static int check_launch(const char* what) {
 }
 
 // ------------------------------------------------------------------------------------------------ 1-8 rows
-// The exact path's product for one to eight activation rows, fused: y (M, N) = x (M, K) @ W.T with W's rows rebuilt
-// from the file's blocks in registers (raw_unit, bit for bit the values mbq_dequant_raw writes), float32 products and
-// sums, each row read once from HBM instead of written as float32 and read back (reference src/mashbox/ops/__init__.py
-// :574-576, 624-632: dequant, then a float32 dot). Lanes in groups of LPR take one weight row each (4 waves x 64 / LPR
-// rows per block, rows over the grid), a lane the row's 32-value units u = lane % LPR, + LPR, ...; the group's sums
-// meet by shuffles; with U2 a lane has two units' loads in flight. Up to RGV_MAX_M activation rows, one float32 sum
-// each in registers.
-constexpr int RGV_MAX_M = 8;
-template <int T, int LPR, bool U2>
-__global__ __launch_bounds__(256) void raw_gemv_kernel(const uint8_t* __restrict__ raw, const uint16_t* __restrict__ x,
-                                                       int M, int N, int K, void* __restrict__ y, int out_bf16) {
-    constexpr int RPB = 256 / LPR;                                       // rows per block
-    const int lane = threadIdx.x & (LPR - 1);
-    const int U = K >> 5;
-    const int64_t rb = raw_row_bytes<T>(K);
-    for (int64_t n = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR; n < N; n += (int64_t)gridDim.x * RPB) {
-        float acc[RGV_MAX_M];
+// Each lane takes one 32-value unit at a time and multiplies it with up to MR activation rows: the types of codes
+// (raw_coded) as bfloat16 pairs with v_dot2_f32_bf16, float32 sums of exact products that the scale multiplies once (a unit
+// that meets a scale, an activation or a sum that is not finite: value by value); the others (F16, F32, TQ1_0) value by value with float32 FMAs, a unit's
+// sum added to the row's. Bound: the vector work (2.5 to 4 instructions per value at one row) and, below about 20 MB, the
+// launch's fill and drain. Against a float64 product it is off by 0.6e-7 to 1.5e-7 (one to eight rows, K 512 to 17408).
+//
+// 8 lanes take 8 consecutive units of a weight row (a super-block of the 256-value types: lane j always its sub-block j, so
+// the shifts of its codes and scales are the lane's constants), a wave 8 rows. The RV_W waves of a block take the 8-unit
+// steps of the same rows in turn (KS of them) or other rows. x is staged once per block in LDS as it comes, RV_X1 or RV_X
+// bytes at a time, a super-block's 16-byte pieces in the order [piece][unit], which the 8 lanes read as 128 consecutive
+// bytes. The bytes of the next step are in flight while a step computes.
+//
+// One row, us (before: 16 to 64 lanes per row, the blocks read a byte or a dword at a time): Q3_K 34816 x 5120 82 -> 27,
+// 5120 x 17408 56 -> 17, 8192 x 5120 24 -> 9.6; IQ4_XS 112 -> 29, 60 -> 18; Q5_0 59 -> 35, 28 -> 21; F16 63 -> 60. Four
+// rows: Q3_K 34816 x 5120 128 -> 43. Two rows of weights per lane (half the LDS reads of x) ran 2 % faster on 34816 rows and
+// 10-20 % slower below 8192, 4 waves per block 5-15 % slower at 5120 x 17408: neither is kept.
+constexpr int RV_W = 8, RV_X1 = 40 * 1024, RV_X = 64 * 1024;
+
+// a step's bytes in flight: a 16-byte piece of a super-block (raw_shared), else the unit itself
+template <int T, bool SH = raw_shared<T>()> struct RawFlight { RawRegs<T> u; };
+template <int T> struct RawFlight<T, true> { u32x4 p; };
+
+template <int T, int MR>
+__global__ __launch_bounds__(64 * RV_W) void raw_gemv_kernel(const uint8_t* __restrict__ raw, const uint16_t* __restrict__ x, int M,
+                                                             int N, int K, void* __restrict__ y, int out_bf16, int KS, int KC) {
+    constexpr bool SH = raw_shared<T>();
+    extern __shared__ __align__(16) uint16_t xs[];                       // [M][KC], the waves' sums, their super-blocks
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 7;
+    const int U = K >> 5, ks = wave % KS, RB = RV_W / KS * 8;            // RB: rows of the block
+    const int n = blockIdx.x * RB + wave / KS * 8 + (lane >> 3);
+    float* const red = reinterpret_cast<float*>(xs + M * KC);            // [wave][8 rows][MR]
+    uint8_t* const sb = reinterpret_cast<uint8_t*>(red + RV_W * 8 * MR) + (wave * 8 + (lane >> 3)) * RAW_SLOT;
+    const uint8_t* row = raw + (int64_t)(n < N ? n : N - 1) * raw_row_bytes<T>(K);
+    float acc[MR];
 #pragma unroll
-        for (int m = 0; m < RGV_MAX_M; ++m) acc[m] = 0.f;
-        const uint8_t* row = raw + n * rb;
-        for (int u0 = lane; u0 < U; u0 += (U2 ? 2 : 1) * LPR)
+    for (int m = 0; m < MR; ++m) acc[m] = 0.f;
+
+    for (int c0 = 0; c0 < K; c0 += KC) {
+        const int kc = K - c0 < KC ? K - c0 : KC, steps = (kc + 255) >> 8, u0 = c0 >> 5;
+        RawFlight<T> fl;
+        auto load = [&](int i) {                                         // past the end: the last unit again
+            const int u = u0 + 8 * (i < steps ? i : steps - 1) + j;
+            if constexpr (SH) fl.p = raw_part<T>(row, u >> 3, j);
+            else raw_load<T>(fl.u, row, u < U ? u : U - 1);
+        };
+        load(ks);
+        if (c0) __syncthreads();                                         // the last chunk's x has been read
+        for (int q = threadIdx.x; q < M * (kc >> 3); q += 64 * RV_W) {
+            const int m = q / (kc >> 3), p = q % (kc >> 3);              // piece p: unit p / 4, its piece p % 4
+            st16(xs + m * KC + (p >> 5) * 256 + ((p & 3) * 8 + ((p >> 2) & 7)) * 8, ld16(x + (int64_t)m * K + c0 + 8 * p));
+        }
+        __syncthreads();
+        for (int i = ks; i < steps; i += KS) {
+            RawRegs<T> cur;
+            if constexpr (SH) {
+                st16(sb + 16 * j, fl.p);
+                __builtin_amdgcn_wave_barrier();                         // a wave's LDS accesses complete in order
+                raw_take<T>(cur, sb, j);
+                __builtin_amdgcn_wave_barrier();
+            } else {
+                cur = fl.u;
+            }
+            load(i + KS);
+            const int u = u0 + 8 * i + j;
+            if (u >= U) continue;
+            const RawScales sc = raw_scales<T>(cur, u);
+            const uint16_t* xp = xs + i * 256 + j * 8;
+            float d[MR];                                                 // the unit's sums
 #pragma unroll
-        for (int uu = 0; uu < (U2 ? 2 : 1); ++uu) {
-            const int u = u0 + uu * LPR;
-            if (u >= U) break;
-            float v[32];
-            raw_unit<T>(row, u, v);
+            for (int m = 0; m < MR; ++m) d[m] = 0.f;
+            bool done = false;
+            if constexpr (raw_coded<T>()) {
+                constexpr int HV = T == T_Q2_K || T == T_Q3_K || T == T_NVFP4 ? 2 : 1;       // scales of a unit
 #pragma unroll
-            for (int m = 0; m < RGV_MAX_M; ++m) {
-                if (m < M) {
-                    const u32x4* xp = reinterpret_cast<const u32x4*>(x + (int64_t)m * K + 32 * u);
+                for (int h = 0; h < HV; ++h) {
+                    float t[MR], sx[MR];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const u32x4 q = xp[c];
+                    for (int m = 0; m < MR; ++m) t[m] = sx[m] = 0.f;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            acc[m] = __builtin_fmaf(__uint_as_float(q[e] << 16), v[8 * c + 2 * e], acc[m]);
-                            acc[m] = __builtin_fmaf(__uint_as_float(q[e] & 0xFFFF0000u), v[8 * c + 2 * e + 1], acc[m]);
+                    for (int s = h * (4 / HV); s < (h + 1) * (4 / HV); ++s) {
+                        uint32_t p[4];
+                        raw_pairs<T>(cur, u, s, p);
+#pragma unroll
+                        for (int m = 0; m < MR; ++m) {
+                            if (MR > 1 && m >= M) break;
+                            const u32x4 q = ld16(xp + m * KC + s * 64);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                if constexpr (raw_min<T>()) sx[m] = dot2(BF16_ONES, q[e], sx[m]);
+                                t[m] = dot2(p[e], q[e], t[m]);
+                            }
                         }
+                    }
+#pragma unroll
+                    for (int m = 0; m < MR; ++m) {
+                        d[m] = __builtin_fmaf(sc.s[h], t[m], d[m]);
+                        if constexpr (raw_min<T>()) d[m] = __builtin_fmaf(sc.b[h], sx[m], d[m]);
+                    }
+                }
+                float f = 0.f;                                           // a non-finite scale, activation or sum makes it NaN
+#pragma unroll
+                for (int m = 0; m < MR; ++m) f = __builtin_fmaf(0.f, d[m], f);
+                done = f == 0.f && raw_finite<T>(sc);
+            }
+            if (!done) {
+#pragma unroll
+                for (int m = 0; m < MR; ++m) d[m] = 0.f;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    float v[8];
+                    raw_vals<T>(cur, sc, u, s, v);
+#pragma unroll
+                    for (int m = 0; m < MR; ++m) {
+                        if (MR > 1 && m >= M) break;
+                        const u32x4 q = ld16(xp + m * KC + s * 64);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            d[m] = __builtin_fmaf(__uint_as_float((e & 1) ? q[e >> 1] & 0xFFFF0000u : q[e >> 1] << 16), v[e], d[m]);
                     }
                 }
             }
+#pragma unroll
+            for (int m = 0; m < MR; ++m) acc[m] += d[m];
         }
+    }
 #pragma unroll
-        for (int m = 0; m < RGV_MAX_M; ++m)
-#pragma unroll
-            for (int off = LPR / 2; off >= 1; off >>= 1) acc[m] += __shfl_xor(acc[m], off, LPR);
-        if (lane == 0) {
-#pragma unroll
-            for (int m = 0; m < RGV_MAX_M; ++m) {
-                if (m < M) {
-                    if (out_bf16) reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)bf16_bits(acc[m]);
-                    else reinterpret_cast<float*>(y)[(int64_t)m * N + n] = acc[m];
-                }
-            }
-        }
+    for (int m = 0; m < MR; ++m) {
+        float t = acc[m];
+        t += dpp_f<0xB1, 0xF>(t);                                        // quad_perm [1,0,3,2]
+        t += dpp_f<0x4E, 0xF>(t);                                        // quad_perm [2,3,0,1]
+        t += dpp_f<0x141, 0xF>(t);                                       // row_half_mirror: the other quad of the 8 lanes
+        if (j == 0) red[(wave * 8 + (lane >> 3)) * MR + m] = t;
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < RB * M; q += 64 * RV_W) {              // the block's rows in order, a row's KS sums in order
+        const int rr = q % RB, m = q / RB, no = blockIdx.x * RB + rr;
+        if (no >= N) continue;
+        const float* p = red + (rr / 8 * KS * 8 + rr % 8) * MR + m;
+        float t = p[0];
+        for (int k = 1; k < KS; ++k) t += p[k * 8 * MR];
+        store_y(y, (int64_t)m * N + no, t, out_bf16);
     }
 }
 
-// Lanes per row by the row's 32-value units U (MI355X, interleaved timings of 16, 32 and 64 lanes, with and without two
-// units in flight, on Q2_K 9728 x 2560, Q3_K 17408 x 5120, IQ4_XS 5120 x 17408, Q5_0 6144 x 5120 at 4 rows and F16
-// 4096 x 4096): short rows (U < 128) 16 lanes, so that a wave holds 4 rows (Q2_K 14.5 -> 10.8 us); the 256-value types,
-// whose units cost the most vector work, 32 lanes up to U = 256 (Q3_K 51.3 -> 46.5 us); else 64, with two units in
-// flight from U = 256 on (IQ4_XS 66.1 -> 60.8 us). Each choice was the fastest or within 2 % of it on those cases.
+// Waves per row: 4, or 8 below 8192 rows, where 4 leave CUs idle (one row, 4 against 8: Q3_K 5120 x 17408 21.5 / 17.0 us,
+// 5120 x 6144 9.6 / 8.4; 34816 x 5120 26.9 / 28.2, 9728 x 2560 7.7 / 7.9); never more than a row has 8-unit steps
+template <int T, int MR>
+static int raw_gemv_m(const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16, hipStream_t s) {
+    int KS = N < 8192 ? 8 : 4;
+    while (KS > 1 && KS * 256 > K) KS /= 2;
+    const int64_t KC = std::min<int64_t>((K + 255) / 256 * 256, (M == 1 ? RV_X1 : RV_X) / (2 * M) / 256 * 256);
+    const size_t lds = (size_t)(M * KC) * 2 + (size_t)RV_W * 8 * (MR * 4 + (raw_shared<T>() ? RAW_SLOT : 0));
+    auto kern = raw_gemv_kernel<T, MR>;
+    static std::atomic<uint64_t> set{0};
+    if (set_lds_limit((const void*)kern, 80 * 1024, set) != hipSuccess) return set_error(MBQ_LAUNCH_FAIL, "raw GEMV: %zu bytes of LDS refused", lds);
+    const int64_t rows = RV_W / KS * 8;
+    kern<<<dim3((unsigned)((N + rows - 1) / rows)), 64 * RV_W, lds, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16, KS, (int)KC);
+    return check_launch("raw GEMV");
+}
+
 template <int T>
-static void raw_gemv_t(const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16,
-                       hipStream_t s) {
-    const int64_t U = K / 32;
-    constexpr bool HEAVY = ggml_block(T).values == 256;
-    if (U < 128)
-        raw_gemv_kernel<T, 16, false><<<dim3((unsigned)((N + 15) / 16)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
-    else if (HEAVY && U < 256)
-        raw_gemv_kernel<T, 32, false><<<dim3((unsigned)((N + 7) / 8)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
-    else if (U < 256)
-        raw_gemv_kernel<T, 64, false><<<dim3((unsigned)((N + 3) / 4)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
-    else
-        raw_gemv_kernel<T, 64, true><<<dim3((unsigned)((N + 3) / 4)), 256, 0, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16);
+static int raw_gemv_t(const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16, hipStream_t s) {
+    if (M == 1) return raw_gemv_m<T, 1>(raw, x, M, N, K, y, out_bf16, s);
+    if (M == 2) return raw_gemv_m<T, 2>(raw, x, M, N, K, y, out_bf16, s);
+    if (M <= 4) return raw_gemv_m<T, 4>(raw, x, M, N, K, y, out_bf16, s);
+    return raw_gemv_m<T, 8>(raw, x, M, N, K, y, out_bf16, s);
 }
 
 int launch_raw_gemv(int t, const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16,
                     hipStream_t s) {
     switch (t) {
-        case T_F32: raw_gemv_t<T_F32>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_F16: raw_gemv_t<T_F16>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_BF16: raw_gemv_t<T_BF16>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_Q4_1: raw_gemv_t<T_Q4_1>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_Q5_0: raw_gemv_t<T_Q5_0>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_Q5_1: raw_gemv_t<T_Q5_1>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_Q2_K: raw_gemv_t<T_Q2_K>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_Q3_K: raw_gemv_t<T_Q3_K>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_IQ4_NL: raw_gemv_t<T_IQ4_NL>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_IQ4_XS: raw_gemv_t<T_IQ4_XS>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_TQ1_0: raw_gemv_t<T_TQ1_0>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_TQ2_0: raw_gemv_t<T_TQ2_0>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_MXFP4: raw_gemv_t<T_MXFP4>(raw, x, M, N, K, y, out_bf16, s); break;
-        case T_NVFP4: raw_gemv_t<T_NVFP4>(raw, x, M, N, K, y, out_bf16, s); break;
-        default: return set_error(MBQ_BAD_ARG, "raw GEMV: no kernel for ggml type %d (kernel types run on their planes)", t);
+#define RAW_CASE(T) case T: return raw_gemv_t<T>(raw, x, M, N, K, y, out_bf16, s);
+        RAW_CASE(T_F32) RAW_CASE(T_F16) RAW_CASE(T_BF16) RAW_CASE(T_Q4_1) RAW_CASE(T_Q5_0) RAW_CASE(T_Q5_1) RAW_CASE(T_Q2_K)
+        RAW_CASE(T_Q3_K) RAW_CASE(T_IQ4_NL) RAW_CASE(T_IQ4_XS) RAW_CASE(T_TQ1_0) RAW_CASE(T_TQ2_0) RAW_CASE(T_MXFP4) RAW_CASE(T_NVFP4)
+#undef RAW_CASE
     }
-    return check_launch("raw GEMV");
+    return set_error(MBQ_BAD_ARG, "raw GEMV: no kernel for ggml type %d (kernel types run on their planes)", t);
 }
-
 
 // ------------------------------------------------------------------------------------- more rows: a bfloat16-split GEMM
 // The float32 product on the bfloat16 matrix cores. x is bfloat16 as it comes; every weight value is the exact sum of

@@ -309,6 +309,8 @@ __device__ __forceinline__ RawScales raw_scales(const RawRegs<T>& r, int u) {
         o.s[0] = o.s[1] = f16f(r.w[4]) * (float)((int)(lo | (hi << 4)) - 32);
     } else if constexpr (T == T_TQ2_0) {
         o.s[0] = o.s[1] = f16f(r.w[8]);
+    } else if constexpr (T == T_BF16) {
+        o.s[0] = o.s[1] = 1.f;
     }
     return o;
 }
@@ -370,6 +372,118 @@ __device__ __forceinline__ void raw_vals(const RawRegs<T>& r, const RawScales& s
             if constexpr (MIN) v[e] = __builtin_fmaf(sc.s[s >> 1], (float)(b & 0xFFu), sc.b[s >> 1]);
             else v[e] = sc.s[s >> 1] * (float)(int8_t)b;
         }
+    }
+}
+
+// ------------------------------------------------------------------------------- codes as bfloat16 pairs
+// For the types whose value is scale * code (+ offset) with an integer code of at most 8 significant bits: the codes of
+// values 8s .. 8s + 7 as four bfloat16 pairs, exact, so that a unit's products with x sum unscaled (v_dot2_f32_bf16) and the
+// scale multiplies the sum of 16 or 32. BF16's values are their own codes (scale 1). Codes of up to 16 values come from byte
+// tables of their bfloat16 halves (a byte permute per 4 codes each), the others through a float32 conversion.
+template <int T>
+__host__ __device__ constexpr bool raw_coded() { return T != T_F32 && T != T_F16 && T != T_TQ1_0; }
+template <int T>
+__host__ __device__ constexpr bool raw_min() { return T == T_Q4_1 || T == T_Q5_1 || T == T_Q2_K; }
+
+// bfloat16 bits of a small integer; entries 4i .. 4i + 3 of a table of them: their low (b = 0) or high (1) bytes
+__host__ __device__ constexpr uint32_t bf16_int(int v) {
+    uint32_t m = (uint32_t)(v < 0 ? -v : v), e = 0;
+    if (m == 0) return 0;
+    while (m >> (e + 1)) ++e;
+    return (v < 0 ? 0x8000u : 0u) | ((127u + e) << 7) | ((e <= 7 ? m << (7 - e) : m >> (e - 7)) & 0x7Fu);
+}
+struct CodeTable { uint32_t b[2][4]; };
+template <int N>
+__host__ __device__ constexpr CodeTable code_table(const int (&v)[N]) {
+    CodeTable t{};
+    for (int i = 0; i < N; ++i)
+        for (int h = 0; h < 2; ++h) t.b[h][i >> 2] |= ((bf16_int(v[i]) >> (8 * h)) & 0xFFu) << (8 * (i & 3));
+    return t;
+}
+template <int T>
+__host__ __device__ constexpr CodeTable raw_table() {
+    constexpr int q2[4] = {0, 1, 2, 3}, q3[8] = {-4, -3, -2, -1, 0, 1, 2, 3}, tq[4] = {-1, 0, 1, 2};
+    constexpr int iq[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
+    constexpr int fp[16] = {0, 1, 2, 3, 4, 6, 8, 12, 0, -1, -2, -3, -4, -6, -8, -12};
+    constexpr int q4[16] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15};
+    return T == T_Q2_K ? code_table(q2) : T == T_Q3_K ? code_table(q3) : T == T_TQ2_0 ? code_table(tq)
+         : T == T_Q4_1 ? code_table(q4) : T == T_MXFP4 || T == T_NVFP4 ? code_table(fp) : code_table(iq);
+}
+
+template <int T>
+__device__ __forceinline__ void raw_pairs(const RawRegs<T>& r, int u, int s, uint32_t p[4]) {
+    static_assert(raw_coded<T>(), "a type of codes");
+    const int j = u & 7;
+    if constexpr (T == T_BF16) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = r.w[4 * s + i];
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {                     // values 8s + 4h .. + 3
+            uint32_t lo, hi;
+            if constexpr (T == T_Q2_K || T == T_Q3_K || T == T_TQ2_0) {
+                constexpr CodeTable t = raw_table<T>();
+                uint32_t c = (r.w[2 * s + h] >> (2 * (j & 3))) & 0x03030303u;
+                if constexpr (T == T_Q3_K) c |= ((r.w[8 + 2 * s + h] >> j) & 0x01010101u) << 2;
+                lo = __builtin_amdgcn_perm(t.b[0][1], t.b[0][0], c);
+                hi = __builtin_amdgcn_perm(t.b[1][1], t.b[1][0], c);
+            } else if constexpr (T == T_Q5_0 || T == T_Q5_1) {
+                uint32_t c = (r.w[2 * (s & 1) + h] >> (4 * (s >> 1))) & 0x0F0F0F0Fu;
+                const uint32_t qh = T == T_Q5_1 ? r.w[5] : __builtin_amdgcn_alignbit(r.w[5], r.w[4], 16);
+                c |= spread4(qh >> (8 * s + 4 * h)) << 4;
+                if constexpr (T == T_Q5_0) c = (c + 0x70707070u) ^ 0x80808080u;
+                p[2 * h] = T == T_Q5_0 ? i8_pair(c, 0) : u8_pair(c, 0);
+                p[2 * h + 1] = T == T_Q5_0 ? i8_pair(c, 1) : u8_pair(c, 1);
+                continue;
+            } else {
+                constexpr CodeTable t = raw_table<T>();
+                const uint32_t c = T == T_NVFP4 ? (r.w[2 * (s >> 1) + h] >> (4 * (s & 1))) & 0x0F0F0F0Fu
+                                                : (r.w[2 * (s & 1) + h] >> (4 * (s >> 1))) & 0x0F0F0F0Fu;
+                const uint32_t i = c & 0x07070707u, sel = ((c >> 1) & 0x04040404u) | 0x03020100u;
+                lo = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t.b[0][3], t.b[0][2], i), __builtin_amdgcn_perm(t.b[0][1], t.b[0][0], i), sel);
+                hi = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t.b[1][3], t.b[1][2], i), __builtin_amdgcn_perm(t.b[1][1], t.b[1][0], i), sel);
+            }
+            p[2 * h] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+            p[2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+        }
+    }
+}
+
+// whether a unit's values, where their scales are finite, are finite themselves (MXFP4's largest scales overflow: 12 * 2^125)
+template <int T>
+__device__ __forceinline__ bool raw_finite(const RawScales& sc) {
+    if constexpr (T == T_MXFP4) return sc.s[0] <= 0x1p124f;
+    else return true;
+}
+
+// ------------------------------------------------------------------------- a super-block, shared by 8 lanes
+// The 2- and 3-bit types' super-blocks, whose bytes several of their 8 units share: 8 lanes load one with a 16-byte load
+// each (raw_part: the block's 16-byte pieces, the last one ending with the block) and leave it in LDS, RAW_SLOT bytes a
+// super-block (the padding spreads 8 of them over the banks), from where each lane takes its unit's registers (raw_take).
+template <int T>
+__host__ __device__ constexpr bool raw_shared() { return T == T_Q2_K || T == T_Q3_K || T == T_TQ2_0; }
+constexpr int RAW_SLOT = 144;
+template <int T>
+__device__ __forceinline__ u32x4 raw_part(const uint8_t* __restrict__ row, int sb, int j) {
+    constexpr int NB = T == T_Q2_K ? 84 : T == T_Q3_K ? 110 : 66;
+    return *reinterpret_cast<const u32x4_u*>(row + (int64_t)sb * NB + (16 * j < NB - 16 ? 16 * j : NB - 16));
+}
+template <int T>
+__device__ __forceinline__ void raw_take(RawRegs<T>& r, const uint8_t* slot, int j) {
+    constexpr int NB = T == T_Q2_K ? 84 : T == T_Q3_K ? 110 : 66, LAST = (NB - 1) / 16 * 16;   // the last piece's place
+    constexpr int Q = T == T_Q2_K ? 16 : T == T_Q3_K ? 32 : 0;
+    const u32x4 a = ld16(slot + Q + 32 * (j >> 2)), b = ld16(slot + Q + 16 + 32 * (j >> 2));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.w[i] = a[i], r.w[4 + i] = b[i];
+    if constexpr (T == T_Q3_K) {
+        const u32x4 c = ld16(slot), d = ld16(slot + 16), e = ld16(slot + LAST);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r.w[8 + i] = c[i], r.w[12 + i] = d[i], r.w[16 + i] = e[i];
+    } else if constexpr (T == T_Q2_K) {
+        r.w[8] = *reinterpret_cast<const uint32_t*>(slot + LAST + 12);
+        r.w[9] = *reinterpret_cast<const uint16_t*>(slot + 2 * j);
+    } else {
+        r.w[8] = *reinterpret_cast<const uint32_t*>(slot + LAST + 12) >> 16;
     }
 }
 

@@ -20,6 +20,12 @@ from tests.test_gpu_raw_types import NAME, _weights
 TOL = 1e-6
 
 
+def _bound(x, w, ref):
+    """TOL of the result's norm, or of the norm that random signs would give it (a few outputs may cancel by chance)"""
+    typical = 1.25 * float((x.double().abs() @ w.double().abs().T).norm()) / w.shape[1] ** 0.5
+    return TOL * max(float(ref.norm()), typical)
+
+
 def _gemm_raw(t, raw, x, n, k, dtype=torch.float32):
     m = x.shape[0]
     y = torch.full((m, n), 7.0, dtype=dtype, device=x.device)
@@ -52,10 +58,11 @@ def test_gemm_raw_against_the_exact_product(t, m, n, k, cuda):
     k = -(-k // max(32, R.TYPES[t][1])) * max(32, R.TYPES[t][1])
     raw = torch.from_numpy(_weights(t, n, k, 31 * t + m)).to(cuda)
     x = torch.from_numpy(np.random.default_rng(m + n).standard_normal((m, k)).astype(np.float32)).to(cuda).to(torch.bfloat16)
-    ref = x.double() @ OPS._raw_dequant(raw, t, n, k).double().T
+    w = OPS._raw_dequant(raw, t, n, k)
+    ref = x.double() @ w.double().T
     y = _gemm_raw(t, raw, x, n, k)
     assert bool(torch.isfinite(y).all())
-    assert float((y.double() - ref).norm()) <= TOL * float(ref.norm())
+    assert float((y.double() - ref).norm()) <= _bound(x, w, ref)
     assert torch.equal(_gemm_raw(t, raw, x, n, k).view(torch.int32), y.view(torch.int32))
     yb = _gemm_raw(t, raw, x, n, k, torch.bfloat16)
     assert torch.equal(yb.view(torch.int16), y.to(torch.bfloat16).view(torch.int16))
@@ -120,3 +127,48 @@ def test_argument_checks():
     assert lib.mbq_gemm_raw(R.Q2_K, None, None, 1 << 20, 1 << 20, 256, None, 0, None, 0, None) < 0   # 2^40 outputs
     assert lib.mbq_gemm_raw(R.Q2_K, None, None, 0, 8, 256, None, 0, None, 0, None) == 0
     assert lib.mbq_gemm_raw_work(-1, 8, 256) < 0 and lib.mbq_gemm_raw_work(0, 8, 256) == 0
+
+
+# --------------------------------------------------------------------------------------------- 1-8 rows (mbq_matmul_raw)
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", R.EXACT_ONLY, ids=NAME.get)
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (1, 8200, 256), (2, 63, 544), (4, 9, 17408), (5, 130, 8448), (8, 8195, 512)])
+def test_decode_rows_against_the_exact_product(t, m, n, k, cuda):
+    """1 to 8 waves per row, rows past a block, a K of half a super-block, x in one or several LDS stages; float32 sums as
+    above: relative 2-norm 1e-6"""
+    from tests.test_gpu_raw_types import _matmul_raw
+    k = -(-k // max(32, R.TYPES[t][1])) * max(32, R.TYPES[t][1])
+    raw = torch.from_numpy(_weights(t, n, k, 13 * t + m)).to(cuda)
+    x = torch.from_numpy(np.random.default_rng(k + n).standard_normal((m, k)).astype(np.float32)).to(cuda).to(torch.bfloat16)
+    w = OPS._raw_dequant(raw, t, n, k)
+    ref = x.double() @ w.double().T
+    y = _matmul_raw(t, raw, x, n, k, False)
+    assert float((y.double() - ref).norm()) <= _bound(x, w, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", R.EXACT_ONLY, ids=NAME.get)
+def test_decode_rows_on_any_bytes(t, cuda):
+    """blocks of random bytes, non-finite and overflowing scales (values) among them, and non-finite activations: inf, -inf
+    and NaN where the float64 product of the rebuilt values has them, wherever no float32 sum can overflow on the way"""
+    from tests.test_gpu_raw_types import _matmul_raw
+    k, n = 512, 700
+    rng = np.random.default_rng(40 + t)
+    raw = _weights(t, n, k, 5).copy()
+    blocks = raw.reshape(n, -1, R.TYPES[t][2])
+    for row in range(0, n, 2):
+        if t == R.MXFP4:
+            blocks[row, rng.integers(blocks.shape[1]), 0] = rng.integers(246, 256)
+        else:
+            blocks[row, rng.integers(blocks.shape[1])] = rng.integers(0, 256, blocks.shape[2], dtype=np.uint8)
+    raw_d = torch.from_numpy(raw).to(cuda)
+    w = OPS._raw_dequant(raw_d, t, n, k).cpu().double()
+    x = torch.from_numpy((rng.standard_normal((3, k)) * 2.0 ** -10).astype(np.float32)).to(torch.bfloat16)
+    x[1, 5], x[2, 7] = float("inf"), float("nan")
+    ref = x.double() @ w.T
+    y = _matmul_raw(t, raw_d, x.to(cuda), n, k, False).cpu().double()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(y[inf], ref[inf])
+    f = torch.isfinite(ref)
+    assert f.any() and bool(((y[f] - ref[f]).abs() <= 1e-5 * (x[0].double().abs() @ w.nan_to_num(0, 0, 0).abs().T).expand(3, n)[f] + 1e-30).all())
