@@ -154,6 +154,11 @@ int mbq_dequant(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* 
 int mbq_dequant_rows(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers,
                      int64_t N, int64_t K, const int32_t* rows_dev, int64_t count, float* w_dev, void* stream);
 
+/* mbq_dequant_rows for ids as a caller holds them, without a pass over them first: int32 or int64 (id_bytes 4 or 8), an id
+ * below zero counting from the end (N added, the sum taken as 32 bits, N added again if still below zero), then clamped. */
+int mbq_lookup_rows(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers,
+                    int64_t N, int64_t K, const void* ids_dev, int id_bytes, int64_t count, float* w_dev, void* stream);
+
 /* W (rows, cols) float32 straight from the file's blocks raw_dev (rows, row_bytes) in HBM, no planes: the exact path's
  * rebuild, bit for bit the reference dequantization (NaN where it has NaN), for every type mbq_has_raw_type names
  * (the float types take any cols; a block type whole blocks). Replaces dequant(raw, t, cols) of reference

@@ -5,6 +5,8 @@ import ctypes
 import os
 import threading
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("MBQ_LIB", os.path.join(HERE, "libmbq.so"))
 
@@ -33,6 +35,8 @@ _SIGS = {
                                _c.c_void_p, _c.c_void_p]),
     "mbq_dequant_rows": (_c.c_int, [_c.c_int, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64,
                                     _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_void_p]),
+    "mbq_lookup_rows": (_c.c_int, [_c.c_int, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64,
+                                   _c.c_void_p, _c.c_int, _c.c_int64, _c.c_void_p, _c.c_void_p]),
     "mbq_dequant_raw": (_c.c_int, [_c.c_int, _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_void_p, _c.c_void_p]),
     "mbq_matmul_raw": (_c.c_int, [_c.c_int, _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_void_p, _c.c_int,
                                   _c.c_void_p]),
@@ -105,8 +109,16 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
-def check(rc: int, what: str) -> int:
+def current_stream() -> int:
+    """the hipStream_t of torch's current stream on the current device (torch.cuda.current_stream().cuda_stream, without
+    the Stream object: 0.2 us of host time against 2.9)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def check(rc: int, what) -> int:
+    """rc, or an MbqError when it is an error code; `what`: the call, as text or as a function that gives it"""
     if rc < 0:
+        what = what() if callable(what) else what
         msg = lib().mbq_last_error().decode(errors="replace")
         raise MbqError(f"{what}: {msg} (code {rc})")
     return rc

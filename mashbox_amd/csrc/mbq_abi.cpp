@@ -244,18 +244,30 @@ int mbq_dequant(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* 
     Args a{};
     if (int rc = plane_args(t, planes_dev, layer, layer_dev, nlayers, N, K, &a)) return rc;
     if (!w_dev || !aligned16(w_dev)) return set_error(MBQ_BAD_ARG, "w is NULL or not 16-byte aligned");
-    return launch_dequant(t, a, w_dev, nullptr, 0, reinterpret_cast<hipStream_t>(stream));
+    return launch_dequant(t, a, w_dev, nullptr, 0, 0, reinterpret_cast<hipStream_t>(stream));
 }
 
-int mbq_dequant_rows(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers,
-                     int64_t N, int64_t K, const int32_t* rows_dev, int64_t count, float* w_dev, void* stream) {
+static int dequant_rows(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers, int64_t N,
+                        int64_t K, const void* rows_dev, int ids, int64_t count, float* w_dev, void* stream) {
     if (t == T_I8T) return set_error(MBQ_BAD_ARG, "int8 planes have no dequant: their values are the int8 quants, scaled per row after the dot");
     Args a{};
     if (int rc = plane_args(t, planes_dev, layer, layer_dev, nlayers, N, K, &a)) return rc;
     if (count < 0 || count > INT32_MAX) return set_error(MBQ_BAD_ARG, "%lld rows", (long long)count);
     if (count == 0) return MBQ_OK;
     if (!rows_dev || !w_dev || !aligned16(w_dev)) return set_error(MBQ_BAD_ARG, "rows or w is NULL, or w not 16-byte aligned");
-    return launch_dequant(t, a, w_dev, rows_dev, count, reinterpret_cast<hipStream_t>(stream));
+    return launch_dequant(t, a, w_dev, rows_dev, ids, count, reinterpret_cast<hipStream_t>(stream));
+}
+
+int mbq_dequant_rows(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers,
+                     int64_t N, int64_t K, const int32_t* rows_dev, int64_t count, float* w_dev, void* stream) {
+    return dequant_rows(t, planes_dev, layer, layer_dev, nlayers, N, K, rows_dev, 0, count, w_dev, stream);
+}
+
+int mbq_lookup_rows(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers,
+                    int64_t N, int64_t K, const void* ids_dev, int id_bytes, int64_t count, float* w_dev, void* stream) {
+    if (id_bytes != 4 && id_bytes != 8) return set_error(MBQ_BAD_ARG, "ids of %d bytes (int32 or int64)", id_bytes);
+    if (reinterpret_cast<uintptr_t>(ids_dev) % (uintptr_t)id_bytes) return set_error(MBQ_BAD_ARG, "misaligned ids");
+    return dequant_rows(t, planes_dev, layer, layer_dev, nlayers, N, K, ids_dev, id_bytes == 4 ? 1 : 2, count, w_dev, stream);
 }
 
 int mbq_dequant_raw(int t, const uint8_t* raw_dev, int64_t rows, int64_t cols, float* w_dev, void* stream) {

@@ -18,11 +18,10 @@ import ctypes
 import numpy as np
 import torch
 
-from ._lib import I8T, OUT_BF16, OUT_F32, check, lib
+from ._lib import I8T, OUT_BF16, OUT_F32, check, current_stream, lib
 
 
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+_stream = current_stream
 
 
 class Int8Planes:
@@ -121,18 +120,21 @@ def _planes_linear(x: torch.Tensor, p: Int8Planes, layer, f32: bool) -> torch.Te
             ld = layer.reshape(()).to(torch.int32)
         else:
             lh = int(layer)
-    lead = tuple(x.shape[:-1])
-    m = 1
-    for v in lead:
-        m *= int(v)
-    y = torch.empty(lead + (p.N,), dtype=torch.float32 if f32 else torch.bfloat16, device=p.buf.device)
+    y = torch.empty((*x.shape[:-1], p.N), dtype=torch.float32 if f32 else torch.bfloat16, device=p.buf.device)
+    m = x.numel() // p.K
     if m == 0:
         return y.zero_()
-    x2 = x.reshape(m, p.K).to(p.buf.device).contiguous()
-    check(lib().mbq_matmul(I8T, ctypes.c_void_p(p.buf.data_ptr()), lh, None if ld is None else ctypes.c_void_p(ld.data_ptr()),
-                           nl, ctypes.c_void_p(x2.data_ptr()), m, p.N, p.K, ctypes.c_void_p(y.data_ptr()),
-                           OUT_F32 if f32 else OUT_BF16, _stream()), f"int8 linear {p}")
+    x = _rows(x, p.buf)
+    check(lib().mbq_matmul(I8T, p.buf.data_ptr(), lh, None if ld is None else ld.data_ptr(), nl, x.data_ptr(), m, p.N, p.K,
+                           y.data_ptr(), OUT_F32 if f32 else OUT_BF16, _stream()), lambda: f"int8 linear {p}")
     return y
+
+
+def _rows(x: torch.Tensor, buf: torch.Tensor) -> torch.Tensor:
+    """x contiguous on buf's GPU: x itself when it is that already"""
+    if x.is_cuda and x.is_contiguous() and x.get_device() == buf.get_device():
+        return x
+    return x.reshape(-1, x.shape[-1]).to(buf.device).contiguous()
 
 
 def linear(x: torch.Tensor, w, pj=None, layer=None) -> torch.Tensor:
@@ -158,18 +160,14 @@ def linear(x: torch.Tensor, w, pj=None, layer=None) -> torch.Tensor:
     if s.shape != (n,):
         raise ValueError(f"w['s'] must be ({n},), got {tuple(s.shape)}")
     q = q.contiguous()
-    lead = tuple(x.shape[:-1])
-    m = 1
-    for v in lead:
-        m *= int(v)
     f32 = pj is not None
-    y = torch.empty(lead + (n,), dtype=torch.float32 if f32 else torch.bfloat16, device=q.device)
+    y = torch.empty((*x.shape[:-1], n), dtype=torch.float32 if f32 else torch.bfloat16, device=q.device)
+    m = x.shape[:-1].numel()
     if m == 0:
         y.zero_()
     else:
-        x2 = x.reshape(m, k).to(q.device).contiguous()
-        check(lib().mbq_int8_linear(ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(s.data_ptr()),
-                                    ctypes.c_void_p(x2.data_ptr()), m, n, k, ctypes.c_void_p(y.data_ptr()),
+        x2 = _rows(x, q)
+        check(lib().mbq_int8_linear(q.data_ptr(), s.data_ptr(), x2.data_ptr(), m, n, k, y.data_ptr(),
                                     OUT_F32 if f32 else OUT_BF16, _stream()), "int8 linear")
     if pj is not None:
         return pj(y).to(x.dtype)

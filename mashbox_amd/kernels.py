@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import INT8, OUT_BF16, OUT_F32, Q4_0, Q40T, Q4_K, Q4KT, Q5_K, Q5KT, Q6_K, Q6KT, Q8_0, Q8T, check, lib
+from ._lib import INT8, OUT_BF16, OUT_F32, Q4_0, Q40T, Q4_K, Q4KT, Q5_K, Q5KT, Q6_K, Q6KT, Q8_0, Q8T, check, current_stream, lib
 
 # the types the reference's kernel package gives planes (reference src/mashbox/ops/bundle.py:39)
 TYPES = frozenset({Q4_0, Q8_0, Q4_K, Q5_K, Q6_K})
@@ -41,12 +41,11 @@ picks_layer = True
 version = "0.1.0"
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+_stream = current_stream
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 def row_bytes(t: int, cols: int) -> int:
@@ -231,23 +230,31 @@ def matmul(x: torch.Tensor, p: Planes, layer=None, out_dtype=torch.float32) -> t
         raise ValueError(f"{p} is on the host: move the planes to the GPU (planes.to('cuda'))")
     if p.alt is not None and x.numel() == x.shape[-1]:
         p = p.alt                                     # one activation row: the row-major planes' decode GEMV
-    p, lh, ld, nl = _layer_args(p, layer)
-    lead = tuple(x.shape[:-1])
-    if x.shape[-1] != p.K:
-        raise ValueError(f"x has {x.shape[-1]} columns, the weight {p.K}")
-    m = 1
-    for v in lead:
-        m *= int(v)
-    y = _out(lead + (p.N,), p.buf.device, out_dtype)
+    lh, ld, nl = 0, None, 1
+    if layer is not None or p.lead:
+        p, lh, ld, nl = _layer_args(p, layer)
+    shape = x.shape
+    n, k = p.N, p.K
+    if shape[-1] != k:
+        raise ValueError(f"x has {shape[-1]} columns, the weight {k}")
+    y = _out((*shape[:-1], n), p.buf.device, out_dtype)
+    m = x.numel() // k
     if m == 0:
         return y.zero_()
-    x2 = x.reshape(m, p.K).to(device=p.buf.device, dtype=torch.bfloat16).contiguous()
     od = OUT_BF16 if out_dtype == torch.bfloat16 else OUT_F32
     if out_dtype not in (torch.float32, torch.bfloat16):
         raise ValueError(f"out_dtype {out_dtype}")
-    check(lib().mbq_matmul(p.t, _ptr(p.buf), lh, None if ld is None else _ptr(ld), nl, _ptr(x2), m, p.N, p.K, _ptr(y),
-                           od, _stream()), f"matmul {p}")
+    x = _rows(x, p.buf)
+    check(lib().mbq_matmul(p.t, _ptr(p.buf), lh, None if ld is None else _ptr(ld), nl, _ptr(x), m, n, k, _ptr(y), od,
+                           _stream()), lambda: f"matmul {p}")
     return y
+
+
+def _rows(x: torch.Tensor, buf: torch.Tensor) -> torch.Tensor:
+    """x as contiguous bfloat16 on buf's GPU: x itself when it is that already"""
+    if x.dtype == torch.bfloat16 and x.is_cuda and x.is_contiguous() and x.get_device() == buf.get_device():
+        return x
+    return x.reshape(-1, x.shape[-1]).to(device=buf.device, dtype=torch.bfloat16).contiguous()
 
 
 def dequant(p: Planes, layer=None) -> torch.Tensor:
@@ -274,14 +281,35 @@ def take_rows(p: Planes, ids, layer=None) -> torch.Tensor:
         raise ValueError(f"{p} is on the host: move the planes to the GPU (planes.to('cuda'))")
     ids = torch.as_tensor(ids, device=p.buf.device)
     idx = ids.reshape(-1).to(torch.int32).contiguous()
-    if layer is None and p.lead:
-        raise ValueError(f"{p}: a stack needs layer= (or index it first)")
-    q, lh, ld, nl = (p, 0, None, 1) if layer is None else _layer_args(p, layer)
+    q, lh, ld, nl = _lookup_args(p, layer)
     w = torch.empty((idx.numel(), p.K), dtype=torch.float32, device=p.buf.device)
     check(lib().mbq_dequant_rows(p.t, _ptr(q.buf), lh, None if ld is None else _ptr(ld), nl, p.N, p.K, _ptr(idx),
-                                 idx.numel(), _ptr(w), _stream()), f"take_rows {p}")
+                                 idx.numel(), _ptr(w), _stream()), lambda: f"take_rows {p}")
     return w.reshape(tuple(ids.shape) + (p.K,))
 
 
-__all__ = ["TYPES", "TILED", "LAYOUTS", "take_rows", "Planes", "repack_host", "repack", "matmul", "dequant", "plane_bytes", "kq_covers",
+def _lookup_args(p: Planes, layer):
+    if layer is not None:
+        return _layer_args(p, layer)
+    if p.lead:
+        raise ValueError(f"{p}: a stack needs layer= (or index it first)")
+    return p, 0, None, 1
+
+
+def lookup_rows(p: Planes, ids: torch.Tensor, layer=None) -> torch.Tensor:
+    """take_rows of int32 or int64 ids on the planes' GPU in one launch: an id below zero counts from the end (added N, and
+    N again where the 32-bit sum is still below zero), then clamped"""
+    if not p.buf.is_cuda:
+        raise ValueError(f"{p} is on the host: move the planes to the GPU (planes.to('cuda'))")
+    if ids.dtype not in (torch.int32, torch.int64):
+        raise TypeError(f"ids must be int32 or int64, got {ids.dtype}")
+    ids = ids.to(p.buf.device).contiguous()
+    q, lh, ld, nl = _lookup_args(p, layer)
+    w = torch.empty((*ids.shape, p.K), dtype=torch.float32, device=p.buf.device)
+    check(lib().mbq_lookup_rows(p.t, _ptr(q.buf), lh, None if ld is None else _ptr(ld), nl, p.N, p.K, _ptr(ids),
+                                ids.element_size(), ids.numel(), _ptr(w), _stream()), lambda: f"lookup_rows {p}")
+    return w
+
+
+__all__ = ["TYPES", "TILED", "LAYOUTS", "take_rows", "lookup_rows", "Planes", "repack_host", "repack", "matmul", "dequant", "plane_bytes", "kq_covers",
            "picks_layer", "row_bytes", "INT8", "Q4KT", "Q8T", "Q5KT", "Q6KT", "Q40T"]

@@ -419,8 +419,7 @@ def stack_rows(parts):
 
 
 # ------------------------------------------------------------------------------------------------- the exact path
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+_stream = _lib.current_stream
 
 
 def _raw_dequant(raw2: torch.Tensor, t: int, rows: int, cols: int) -> torch.Tensor:
@@ -454,27 +453,27 @@ def _raw_product(x: torch.Tensor, h: "Raw") -> torch.Tensor | None:
     where it does not apply (other dtypes: the reference multiplies float32 x, not its bfloat16 rounding; sizes past the
     kernels' 32-bit counts; more than 8 rows that something differentiates, transforms or traces)"""
     rows, cols = h.shape[-2:]
-    lead = tuple(x.shape[:-1])
-    m = int(np.prod(lead, dtype=np.int64)) if lead else 1
+    m = x.shape[:-1].numel()
     if (x.dtype != torch.bfloat16 or m < 1 or h.t in (2, 8, 12, 13, 14) or cols % max(32, TYPES[h.t][1])
             or (m > RAW_GEMV_MAX_M and (max(m * cols, m * rows) > 0x7FFFFFFF or not _untraced(x)))):
         return None                                  # (the kernel types' blocks, off the kernels: rebuild and GEMM)
-    blocks = _blocks(h).reshape(rows, -1).contiguous()
-    x2 = x.reshape(m, cols).to(blocks.device).contiguous()
-    y = torch.empty((m, rows), dtype=torch.bfloat16, device=blocks.device)
+    raw = h.raw
+    if raw.dim() != 2 or not raw.is_contiguous() or raw.shape[0] != rows or raw.shape[1] != row_bytes(h.t, cols):
+        raw = _blocks(h).reshape(rows, -1).contiguous()
+    if x.shape[-1] != cols or not x.is_contiguous() or x.get_device() != raw.get_device():
+        x = x.reshape(x.shape[:-1] + (cols,)).to(raw.device).contiguous()
+    y = torch.empty((*x.shape[:-1], rows), dtype=torch.bfloat16, device=raw.device)
     lib = _lib.lib()
-    p = ctypes.c_void_p
     if m <= RAW_GEMV_MAX_M:
-        _lib.check(lib.mbq_matmul_raw(int(h.t), p(blocks.data_ptr()), p(x2.data_ptr()), m, rows, cols, p(y.data_ptr()), 1,
-                                      _stream()), "matmul_raw")
+        _lib.check(lib.mbq_matmul_raw(h.t, raw.data_ptr(), x.data_ptr(), m, rows, cols, y.data_ptr(), 1, _stream()), "matmul_raw")
     else:
-        if x2.data_ptr() % 16:                       # a view at an odd offset: the kernel copies 16 bytes at a time
-            x2 = x2.clone()
+        if x.data_ptr() % 16:                        # a view at an odd offset: the kernel copies 16 bytes at a time
+            x = x.clone()
         nwork = _lib.check(lib.mbq_gemm_raw_work(m, rows, cols), "gemm_raw_work")
-        work = torch.empty(nwork, dtype=torch.uint8, device=blocks.device)
-        _lib.check(lib.mbq_gemm_raw(int(h.t), p(blocks.data_ptr()), p(x2.data_ptr()), m, rows, cols, p(y.data_ptr()), 1,
-                                    p(work.data_ptr()), nwork, _stream()), "gemm_raw")
-    return y.reshape(lead + (rows,))
+        work = torch.empty(nwork, dtype=torch.uint8, device=raw.device)
+        _lib.check(lib.mbq_gemm_raw(h.t, raw.data_ptr(), x.data_ptr(), m, rows, cols, y.data_ptr(), 1, work.data_ptr(), nwork,
+                                    _stream()), "gemm_raw")
+    return y
 
 
 def _exact_matmul(x: torch.Tensor, h: Raw) -> torch.Tensor:
@@ -559,20 +558,29 @@ def dequant(h) -> torch.Tensor:
     return _raw_dequant(flat, h.t, flat.shape[0], cols).reshape(tuple(blocks.shape[:-2]) + (rows, cols))
 
 
+def _from_the_end(ids: torch.Tensor, rows: int) -> torch.Tensor:
+    ids = ids.long()
+    return torch.where(ids < 0, ids + rows, ids)
+
+
 def take_rows(h, ids) -> torch.Tensor:
     """rows `ids` of the weights as float32 (an embedding lookup), exact; an id below zero counts from the end. Only the
     looked-up rows are rebuilt."""
     if isinstance(h, Pick):
         return _on_pick(h, lambda one: take_rows(one, ids))
     rows, cols = h.shape[-2:]
-    ids = torch.as_tensor(ids, device=_device()).long()
-    ids = torch.where(ids < 0, ids + rows, ids)
-    gather = getattr(_KERNELS.module, "take_rows", None)
+    ids = torch.as_tensor(ids, device=_device())
     if isinstance(h, (Packed, At)):
         layer = h.layer if isinstance(h, At) else None
+        lookup = getattr(_KERNELS.module, "lookup_rows", None)
+        if lookup is not None and ids.dtype in (torch.int32, torch.int64):
+            return lookup(h.packed, ids, layer=layer)
+        ids = _from_the_end(ids, rows)
+        gather = getattr(_KERNELS.module, "take_rows", None)
         if gather is not None:
             return gather(h.packed, ids, layer=layer)
         return (dequant(h))[ids]
+    ids = _from_the_end(ids, rows)
     blocks = _blocks(h).reshape(rows, -1)
     picked = blocks[ids.reshape(-1)].contiguous()
     if picked.shape[0] == 0:
