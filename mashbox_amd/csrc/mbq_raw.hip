@@ -25,8 +25,8 @@ static int check_launch(const char* what) {
 // ------------------------------------------------------------------------------------------------ 1-8 rows
 // Each lane takes one 32-value unit at a time and multiplies it with up to MR activation rows: the types of codes
 // (raw_coded) as bfloat16 pairs with v_dot2_f32_bf16, float32 sums of exact products that the scale multiplies once (a unit
-// that meets a scale, an activation or a sum that is not finite: value by value); the others (F16, F32, TQ1_0) value by value with float32 FMAs, a unit's
-// sum added to the row's. Bound: the vector work (2.5 to 4 instructions per value at one row) and, below about 20 MB, the
+// that meets a scale, an activation or a sum that is not finite: value by value); the others (F16, F32, TQ1_0) value by
+// value with float32 FMAs, a unit's sum added to the row's. Bound: the vector work (2.5 to 4 instructions per value at one row) and, below about 20 MB, the
 // launch's fill and drain. Against a float64 product it is off by 0.6e-7 to 1.5e-7 (one to eight rows, K 512 to 17408).
 //
 // 8 lanes take 8 consecutive units of a weight row (a super-block of the 256-value types: lane j always its sub-block j, so
@@ -208,8 +208,8 @@ int launch_raw_gemv(int t, const uint8_t* raw, const uint16_t* x, int64_t M, int
 // rest), so the MFMAs multiply exactly and only their float32 accumulation rounds, as a float32 GEMM's does. Against a
 // float64 product (2-norm, 512 x 4096 x 5120) it is off by 1.5e-7 to 2.7e-7, the rebuild and float32 library GEMM it
 // replaces by 0.7e-6 to 1.3e-6; smaller shapes alike. The float32 GEMM runs at 98 TFLOP/s here; this kernel's MFMAs at
-// 1.25 PFLOP/s, 418 TFLOP/s of the product with three terms, 582 with two, 749 with one (512 rows, 34816 x 5120: IQ4_XS
-// 436 us, Q5_0 313, BF16 244; the rebuild and float32 GEMM 2.2 ms).
+// 1.25 PFLOP/s, 420 TFLOP/s of the product with three terms, 567 with two, 749 with one (512 rows, 34816 x 5120: Q3_K
+// 434 us, F16 322, BF16 244; the rebuild and float32 GEMM 2.2 ms).
 //
 // Tile: 32 BMT activation rows x 256 weight rows, K step 64, 8 waves. Wave w owns weight rows 32w .. 32w + 31 and all
 // the activation rows (BMT accumulators of v_mfma_f32_32x32x16_bf16): its lane l decodes unit l / 32 of the K step of row
@@ -222,9 +222,9 @@ int launch_raw_gemv(int t, const uint8_t* raw, const uint16_t* x, int64_t M, int
 // so that at the next barrier's wait only that DMA may be outstanding: the wait counts DMA instructions alone.
 //
 // The tiles that do not fill a round of the CUs are cut along K into S pieces, each a block of its own, whose float32
-// partials the second kernel adds in piece order. Where an output comes out NaN (a non-finite weight or activation,
-// whose lower terms are inf - inf or meet 0 * inf), it is recomputed value by value, so that it is what the float32
-// product gives.
+// partials the second kernel adds in piece order. An output that is not finite (a non-finite weight or activation, whose
+// lower terms are inf - inf or meet 0 * inf, or a sum past the range) is computed again value by value, so that it is what
+// the float32 product gives.
 constexpr int RG_T = 512, RG_BN = 256, RG_K = 64;
 
 struct RawGemmArgs {
@@ -280,9 +280,66 @@ __device__ __forceinline__ void raw_split(const float v[8], bf16x8_t b[NT]) {
     }
 }
 
+// Types whose 32 values share one scale and whose codes need no more than a bfloat16's 8 bits (raw_factored): one MFMA per
+// code instead of three per value. Both lane halves hold the same unit (half h its values 8h .. + 7 and 16 + 8h .. + 7, the
+// low and high nibbles of bytes 8h .. + 7), so two MFMAs sum a unit alone, unscaled, and 16 FMAs per row tile add scale times
+// that sum to the accumulators, behind the MFMAs of the next two row tiles. A scale that is not finite goes in as NaN. Bound:
+// the FMAs and the decode, about 400 vector instructions against 32 MFMAs of 32 cycles per wave and step. IQ4_XS, 512 rows,
+// against three terms: 34816 x 5120 436 -> 283 us, 5120 x 17408 220 -> 147, 8192 x 5120 115 -> 80; 16 rows 80 -> 57. Error
+// against float64 2.7e-7 -> 1.0e-7. Q5_0, two terms otherwise: 512 rows 313 -> 276 us, 64 rows 78 -> 73, but
+// 5120 x 6144 at 16 rows 21.4 -> 24.5, so from 33 rows.
+template <int T, int BMT>
+__host__ __device__ constexpr bool raw_factored() { return T == T_IQ4_NL || T == T_IQ4_XS || (T == T_Q5_0 && BMT >= 2); }
+template <int T> struct RawHalf { uint32_t q[2][2], h[T == T_IQ4_XS ? 2 : 4]; };     // two units' nibbles; their headers
+
+template <int T>
+__device__ __forceinline__ void raw_half_load(RawHalf<T>& r, const uint8_t* __restrict__ row, int it, int half, int U) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const int u = 2 * it + w < U ? 2 * it + w : U - 1;              // past K: the last unit again (it meets zeros)
+        const uint8_t* b = row + (T == T_IQ4_XS ? (int64_t)(u >> 3) * 136 : (int64_t)u * (T == T_Q5_0 ? 22 : 18));
+        const u32x2 q = *reinterpret_cast<const u32x2_u*>(b + (T == T_IQ4_XS ? 8 + 16 * (u & 7) : T == T_Q5_0 ? 6 : 2) + 8 * half);
+        r.q[w][0] = q[0];
+        r.q[w][1] = q[1];
+        if constexpr (T == T_IQ4_NL) {
+            r.h[w] = *reinterpret_cast<const u16_u*>(b);
+        } else if (T == T_Q5_0 || w == 0) {
+            const u32x2 h = *reinterpret_cast<const u32x2_u*>(b);
+            r.h[2 * w] = h[0];
+            r.h[2 * w + 1] = h[1];
+        }
+    }
+}
+
+// unit w's scale, and its codes as two B operands
+template <int T>
+__device__ __forceinline__ float raw_half_codes(const RawHalf<T>& r, int it, int w, int half, bf16x8_t b[2]) {
+    RawRegs<T> g;
+    g.w[0] = r.q[w][0];
+    g.w[1] = r.q[w][1];
+    g.w[2] = g.w[3] = 0;
+    if constexpr (T == T_IQ4_NL) g.w[4] = r.h[w];
+    else if constexpr (T == T_IQ4_XS) g.w[4] = r.h[0], g.w[5] = r.h[1];
+    else g.w[4] = r.h[2 * w], g.w[5] = r.h[2 * w + 1];
+    if constexpr (T == T_Q5_0) {                                         // the high bits of values 8h .. + 7 and 16 + 8h .. + 7
+        const uint32_t qh = __builtin_amdgcn_alignbit(g.w[5], g.w[4], 16) >> (8 * half);
+        g.w[5] = qh >> 16;
+        g.w[4] = (g.w[4] & 0xFFFFu) | (qh << 16);
+    }
+    const float s = raw_scales<T>(g, 2 * it + w).s[0];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {                                        // raw_pairs' steps 0 and 2: low, high nibbles of w[0], w[1]
+        uint32_t p[4];
+        raw_pairs<T>(g, 0, 2 * k, p);
+        b[k] = __builtin_bit_cast(bf16x8_t, u32x4{p[0], p[1], p[2], p[3]});
+    }
+    return __builtin_fabsf(s) < __builtin_inff() ? s : __builtin_nanf("");
+}
+
 template <int T, int BMT>
 __global__ __launch_bounds__(RG_T, BMT >= 4 || T == T_TQ1_0 ? 2 : 4) void raw_gemm_kernel(const RawGemmArgs g) {
     constexpr int NT = raw_terms<T>(), BM = 32 * BMT, STAGE = BM * RG_K;
+    constexpr bool FACT = raw_factored<T, BMT>();
     constexpr int ND = BMT >= 2 ? BMT / 2 : 1;                           // DMA instructions of a wave per stage
     extern __shared__ __align__(16) uint16_t lds[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
@@ -320,10 +377,14 @@ __global__ __launch_bounds__(RG_T, BMT >= 4 || T == T_TQ1_0 ? 2 : 4) void raw_ge
     for (int r = 0; r < BMT; ++r)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[r][i] = 0.f;
-    RawRegs<T> cur, nxt;
+    std::conditional_t<FACT, RawHalf<T>, RawRegs<T>> cur, nxt;
+    auto load = [&](auto& d, int it) {
+        if constexpr (FACT) raw_half_load<T>(d, row, it < k1 ? it : k1 - 1, half, U);
+        else raw_load<T>(d, row, unit(it));
+    };
     dma(k0, 0);
     asm volatile("" ::: "memory");
-    raw_load<T>(cur, row, unit(k0));
+    load(cur, k0);
     asm volatile("" ::: "memory");
     dma(k0 + 1, 1);
 
@@ -332,24 +393,56 @@ __global__ __launch_bounds__(RG_T, BMT >= 4 || T == T_TQ1_0 ? 2 : 4) void raw_ge
         wait_vm<ND>();                                                    // all but the next stage's DMA has landed
         wait_lgkm0();                                                     // and the last step's reads of the stage DMA fills next
         barrier_nofence();
-        raw_load<T>(nxt, row, unit(it + 1));
+        load(nxt, it + 1);
         asm volatile("" ::: "memory");
         dma(it + 2, st2);
-        const int u = unit(it);
-        const RawScales sc = raw_scales<T>(cur, u);
         const uint16_t* st = lds + st0 * STAGE;
+        if constexpr (FACT) {
+            constexpr int RT = BMT >= 2 ? 2 : 1, NG = 2 * BMT / RT;      // groups of RT row tiles, unit 0's then unit 1's
+            const f32x16_t zero = {};
+            bf16x8_t b[2];
+            float s = 0.f, sp = 0.f;
+            f32x16_t P[2][RT];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            float v[8];
-            raw_vals<T>(cur, sc, u, s, v);
-            bf16x8_t bt[NT], a[BMT];
-            raw_split<NT>(v, bt);
+            for (int i = 0; i <= NG; ++i) {
+                const int w = i / (NG / 2), r0 = i % (NG / 2) * RT;
+                if (i < NG) {
+                    sp = s;
+                    if (r0 == 0) s = raw_half_codes<T>(cur, it, w, half, b);
 #pragma unroll
-            for (int r = 0; r < BMT; ++r) a[r] = __builtin_bit_cast(bf16x8_t, ld16(st + rg_off(32 * r + col, 4 * half + s)));
+                    for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int k = 0; k < NT; ++k)
+                        for (int r = 0; r < RT; ++r) {
+                            const bf16x8_t a = __builtin_bit_cast(bf16x8_t, ld16(st + rg_off(32 * (r0 + r) + col, 4 * w + 2 * k + half)));
+                            P[i & 1][r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[k], k == 0 ? zero : P[i & 1][r], 0, 0, 0);
+                        }
+                } else {
+                    sp = s;
+                }
+                if (i > 0) {
+                    const int q0 = (i - 1) % (NG / 2) * RT;
 #pragma unroll
-                for (int r = 0; r < BMT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r], bt[k], acc[r], 0, 0, 0);
+                    for (int r = 0; r < RT; ++r)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[q0 + r][e] = __builtin_fmaf(sp, P[(i - 1) & 1][r][e], acc[q0 + r][e]);
+                }
+            }
+        } else {
+            const int u = unit(it);
+            const RawScales sc = raw_scales<T>(cur, u);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float v[8];
+                raw_vals<T>(cur, sc, u, s, v);
+                bf16x8_t bt[NT], a[BMT];
+                raw_split<NT>(v, bt);
+#pragma unroll
+                for (int r = 0; r < BMT; ++r) a[r] = __builtin_bit_cast(bf16x8_t, ld16(st + rg_off(32 * r + col, 4 * half + s)));
+#pragma unroll
+                for (int k = 0; k < NT; ++k)
+#pragma unroll
+                    for (int r = 0; r < BMT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r], bt[k], acc[r], 0, 0, 0);
+            }
         }
         cur = nxt;
         st0 = st0 == 2 ? 0 : st0 + 1;
@@ -365,7 +458,7 @@ __global__ __launch_bounds__(RG_T, BMT >= 4 || T == T_TQ1_0 ? 2 : 4) void raw_ge
             for (int i = 0; i < 16; ++i) o[(32 * r + 8 * (i >> 2) + (i & 3)) * RG_BN] = acc[r][i];
         return;
     }
-    uint32_t bad[(BMT + 1) / 2] = {};                                     // the lane's NaN outputs, a bit each
+    uint32_t bad[(BMT + 1) / 2] = {};                                     // the lane's non-finite outputs, a bit each
     auto store = [&](auto bf16) {
 #pragma unroll
         for (int r = 0; r < BMT; ++r)
@@ -374,7 +467,7 @@ __global__ __launch_bounds__(RG_T, BMT >= 4 || T == T_TQ1_0 ? 2 : 4) void raw_ge
                 const int m = m0 + 32 * r + 8 * (i >> 2) + 4 * half + (i & 3);
                 if (m < g.M && n < g.N) {
                     store_y(g.y, (int64_t)m * g.N + n, acc[r][i], decltype(bf16)::value);
-                    bad[r >> 1] |= acc[r][i] != acc[r][i] ? 1u << (16 * (r & 1) + i) : 0u;
+                    bad[r >> 1] |= !(__builtin_fabsf(acc[r][i]) < __builtin_inff()) ? 1u << (16 * (r & 1) + i) : 0u;
                 }
             }
     };
@@ -408,7 +501,7 @@ __global__ __launch_bounds__(256) void raw_reduce_kernel(const RawGemmArgs g, in
         const int n = n0 + i;
         if (n >= g.N) break;
         float f = v[i];
-        if (f != f) f = raw_dot<T>(g.raw + (int64_t)n * raw_row_bytes<T>(g.K), g.x + (int64_t)m * g.K, g.K);
+        if (!(__builtin_fabsf(f) < __builtin_inff())) f = raw_dot<T>(g.raw + (int64_t)n * raw_row_bytes<T>(g.K), g.x + (int64_t)m * g.K, g.K);
         store_y(g.y, (int64_t)m * g.N + n, f, g.out_bf16);
     }
 }

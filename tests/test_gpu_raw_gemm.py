@@ -52,7 +52,7 @@ def test_unit_rows_give_back_the_weights(t, cuda):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("t", R.EXACT_ONLY, ids=NAME.get)
-@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (9, 255, 320), (32, 257, 64), (33, 513, 1280), (64, 70, 4096), (65, 300, 2304),
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (9, 255, 320), (70, 90, 96), (32, 257, 64), (33, 513, 1280), (64, 70, 4096), (65, 300, 2304),
                                    (129, 256, 5120), (257, 1025, 768), (513, 40, 544)])
 def test_gemm_raw_against_the_exact_product(t, m, n, k, cuda):
     k = -(-k // max(32, R.TYPES[t][1])) * max(32, R.TYPES[t][1])
