@@ -224,7 +224,9 @@ int mbq_int8_embed(const int8_t* q_dev, const float* s_dev, int64_t N, int64_t D
  *   MBQ_KERNEL_STREAM  weight-stream kernel, M <= 64 (M <= 4 when the GEMV has no plan: e.g. K = 17408 at 3-4 rows,
  *                      Q8_0 / int8 rows over 24576 values): bm = 16, bn = weight rows per block (64 or 128); from 17
  *                      rows on, a weight of at least 64 rows per CU runs MBQ_KERNEL_TILES instead (automatic plan).
- *   MBQ_KERNEL_TILES   LDS-tile kernel: 256x{256,192,128}, 128x{256,192,128,64}, 64x{256,192,128,64}.
+ *   MBQ_KERNEL_TILES   LDS-tile kernel: 256x{256,192,128}, 128x{256,192,128,64}, 64x{256,192,128,64}. An automatic
+ *                      256x192 plan with splits > 1 splits only the tiles of the last, partial round of the CUs; where
+ *                      it finds no workspace (below) it runs them whole.
  *   MBQ_KERNEL_KGROUP  K-group kernel of tiled planes (MBQ_I8T and the tiled GGUF types) at M <= 64:
  *                      bm = 16, bn = weight rows per block (any count: N is cut into equal ranges that fill the
  *                      CUs, or several rounds of them for a weight of more than about 96 rows per CU), splits = K

@@ -249,6 +249,7 @@ struct GemmArgs {
     int* cnt;                   // S > 1: per-tile arrival counters (zero between launches)
     uint32_t ws_bytes;          // S > 1: bytes of ws
     int fenced;                 // S > 1: ws is cached memory: release / acquire around the exchange
+    int full;                   // sgemm_kernel: tiles run whole; each tile past them is S blocks of kts K steps
 };
 
 // Pipeline of depth P (1 or 3): x is DMA'd P steps ahead into P + 1 LDS stages, weight units are loaded into P + 1
@@ -499,27 +500,31 @@ constexpr size_t SG_LDS = (size_t)(3 * SG_BM + 2 * SG_BN) * GK * sizeof(uint16_t
 constexpr int SG_QS = 104;
 static_assert((size_t)4 * 128 * SG_QS * sizeof(uint16_t) <= SG_LDS && SG_QS % 8 == 0, "output quarters fit the LDS");
 
-template <int T, bool KFULL>
+template <int T, bool KFULL, bool PIECES>
 __global__ __launch_bounds__(GT, 1) void sgemm_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) uint16_t sg_lds[];   // A[3][256][64], B[2][192][64] bfloat16
     uint16_t* const A0 = sg_lds;
     uint16_t* const B0 = sg_lds + 3 * SG_BM * GK;
     const int M = g.M, N = g.N, K = g.K;
 
-    // XCD-aware order, as gemm_kernel
-    const int MT = (M + SG_BM - 1) / SG_BM, NT = (N + SG_BN - 1) / SG_BN, TB = MT * NT;
-    const int b = blockIdx.x, xcd = b & 7, q = TB >> 3, rem = TB & 7;
-    const int tile = xcd * q + min(xcd, rem) + (b >> 3);
+    // XCD-aware order, as gemm_kernel: the whole tiles, then the pieces by K range, so that an XCD's blocks share x and K
+    const int NT = (N + SG_BN - 1) / SG_BN;
+    const bool piece = PIECES && (int)blockIdx.x >= g.full;
+    const int b = piece ? blockIdx.x - g.full : blockIdx.x, TB = piece ? gridDim.x - g.full : g.full;
+    const int xcd = b & 7, q = TB >> 3, rem = TB & 7, at = xcd * q + min(xcd, rem) + (b >> 3);
+    const int rest = piece ? TB / g.S : 1, kp = piece ? at / rest : 0;    // the piece's K range and its place in ws
+    const int tile = piece ? g.full + at - kp * rest : at, pc = (at - kp * rest) * g.S + kp;
     const int m0 = (tile / NT) * SG_BM, n0 = (tile % NT) * SG_BN;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t lo = layer_offset(g.stride, g.layer_dev, g.nlayers);
     const bool ok = lo >= 0;
-    const int KT = (K + GK - 1) / GK, n = ok ? KT : 0;
-    auto k0 = [&](int l) { return min(l, n - 1) * GK; };
+    const int KT = (K + GK - 1) / GK, l0 = kp * g.kts;
+    const int n = !ok ? 0 : piece ? min(g.kts, KT - l0) : KT;             // K steps l0 .. l0 + n - 1
+    auto k0 = [&](int l) { return (l0 + min(l, n - 1)) * GK; };
     auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
     // bfloat16 output rows whose 8-value chunks are 16-byte aligned leave through LDS (the consumers' epilogue)
-    const bool vec = g.out_bf16 && (N & 7) == 0 && (reinterpret_cast<uintptr_t>(g.y) & 15) == 0;
+    const bool vec = !piece && g.out_bf16 && (N & 7) == 0 && (reinterpret_cast<uintptr_t>(g.y) & 15) == 0;
 
     if (wave < 4) {
         // ---------------------------------------------------------------------------------------------- consumer
@@ -565,6 +570,21 @@ __global__ __launch_bounds__(GT, 1) void sgemm_kernel(const GemmArgs g) {
             mfma_drain();
         }
         // lane holds weight row n0 + 96 cn + 32 j + (lane & 31) and activation rows m0 + 128 cm + 32 i + 8 e + 4 (lane >> 5) + r
+        if (piece) {                                               // its partial tile, [256][192] float32
+            const rsrc_t pr = make_rsrc(g.ws + (int64_t)pc * SG_BM * SG_BN, SG_BM * SG_BN * 4);
+            const uint32_t vo = (uint32_t)((cm * 128 + 4 * lh) * SG_BN + br) * 4u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int j = 0; j < 3; ++j)
+                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][4 * e + r]), pr, vo,
+                                                                  (uint32_t)((32 * i + 8 * e + r) * SG_BN + 32 * j) * 4u, 0);
+            return;
+        }
         float scs[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -753,6 +773,24 @@ __global__ __launch_bounds__(GT, 1) void sgemm_kernel(const GemmArgs g) {
     if (vec) barrier_nofence();                                       // the consumers may now write the output tile into LDS
 }
 
+// The tiles past g.full: the S partials of each output added in K order, times the row scale, to y (4 columns a thread).
+// A kernel of its own, so that the pieces exchange nothing while they run.
+template <int T>
+__global__ __launch_bounds__(256) void sgemm_sum_kernel(const GemmArgs g) {
+    const int NT = (g.N + SG_BN - 1) / SG_BN, tile = g.full + blockIdx.y;
+    const int e = (int)(blockIdx.x * 256 + threadIdx.x) * 4, m = (tile / NT) * SG_BM + e / SG_BN, n0 = (tile % NT) * SG_BN + e % SG_BN;
+    if (m >= g.M || n0 >= g.N) return;
+    const int64_t lo = layer_offset(g.stride, g.layer_dev, g.nlayers);
+    const float* p = g.ws + (int64_t)blockIdx.y * g.S * (SG_BM * SG_BN) + e;
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(p);
+    for (int k = 1; k < g.S; ++k) v += *reinterpret_cast<const f32x4_t*>(p + (int64_t)k * (SG_BM * SG_BN));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = n0 + i;
+        if (n < g.N) store_y(g.y, (int64_t)m * g.N + n, lo >= 0 ? v[i] * row_scale<T>(g.srow, g.base + lo, g.sc_off, n) : __builtin_nanf(""), g.out_bf16);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------- workspace
 // Split-K partials and arrival counters: one set per (device, stream), so that split-K calls overlapping in time on two
 // streams of a device (a server's prefill and decode streams) never share partials or counters. A stream's set is
@@ -891,35 +929,47 @@ static int launch_tile(const Args& a, int S, int kts, const Workspace& w, hipStr
     return 0;
 }
 
-template <int T, bool KFULL>
-static int launch_sg(const Args& a, hipStream_t s) {
-    auto kern = sgemm_kernel<T, KFULL>;
+static int64_t sg_tiles(int64_t M, int64_t N) { return ((M + SG_BM - 1) / SG_BM) * ((N + SG_BN - 1) / SG_BN); }
+
+// S = 1: every tile whole; else the tiles past `full` as S pieces of kts K steps, their partials in w
+template <int T, bool KFULL, bool PIECES>
+static int launch_sg_p(const Args& a, int full, int S, int kts, const Workspace& w, hipStream_t s) {
+    auto kern = sgemm_kernel<T, KFULL, PIECES>;
     static std::atomic<uint64_t> lds_set{0};
     if (set_lds_limit((const void*)kern, SG_LDS, lds_set) != hipSuccess)
         return set_error(MBQ_LAUNCH_FAIL, "GEMM: %zu bytes of LDS refused", SG_LDS);
     GemmArgs g{a.base, a.stride, a.layer_dev, a.nlayers, a.sc_off, a.wbytes, a.hi_off, a.d_off, a.srow, a.x, (int)a.M,
-               (int)a.N, (int)a.K, a.y, a.out_bf16, 1, (int)((a.K + GK - 1) / GK), nullptr, nullptr, 0u};
-    const int64_t tiles = ((a.M + SG_BM - 1) / SG_BM) * ((a.N + SG_BN - 1) / SG_BN);
-    kern<<<dim3((unsigned)tiles), GT, SG_LDS, s>>>(g);
+               (int)a.N, (int)a.K, a.y, a.out_bf16, S, kts, w.ws, nullptr, 0u, 0, full};
+    const int64_t rest = sg_tiles(a.M, a.N) - full;
+    kern<<<dim3((unsigned)(full + rest * S)), GT, SG_LDS, s>>>(g);
+    if (rest > 0) sgemm_sum_kernel<T><<<dim3(SG_BM * SG_BN / 1024, (unsigned)rest), 256, 0, s>>>(g);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(MBQ_LAUNCH_FAIL, "GEMM launch: %s", hipGetErrorString(e));
     return 0;
 }
 
-// the 256 x 192 tile without a K split runs the specialized-wave kernel; K-quant rows (multiples of 256 values) always
-// fill whole K steps
+template <int T, bool KFULL>
+static int launch_sg(const Args& a, int full, int S, int kts, const Workspace& w, hipStream_t s) {
+    return S == 1 ? launch_sg_p<T, KFULL, false>(a, full, S, kts, w, s) : launch_sg_p<T, KFULL, true>(a, full, S, kts, w, s);
+}
+
+// the 256 x 192 tile without a K split, or with the pieces of a plan (full >= 0), runs the specialized-wave kernel; K-quant
+// rows (multiples of 256 values) always fill whole K steps
 template <int T, int BM, int BN, int P>
-static int launch_k(const Args& a, int S, int kts, const Workspace& w, hipStream_t s) {
+static int launch_k(const Args& a, int S, int kts, int full, const Workspace& w, hipStream_t s) {
+    const bool sg = BM == SG_BM && BN == SG_BN && (S == 1 || full >= 0);
+    if (S == 1) full = (int)sg_tiles(a.M, a.N);
     if constexpr (kquant(T)) {
-        if (BM == SG_BM && BN == SG_BN && S == 1) return launch_sg<T, true>(a, s);
+        if (sg) return launch_sg<T, true>(a, full, S, kts, w, s);
         return launch_tile<T, BM, BN, P, true>(a, S, kts, w, s);
     } else {
-        if (BM == SG_BM && BN == SG_BN && S == 1) return (a.K % GK == 0) ? launch_sg<T, true>(a, s) : launch_sg<T, false>(a, s);
+        if (sg) return (a.K % GK == 0) ? launch_sg<T, true>(a, full, S, kts, w, s) : launch_sg<T, false>(a, full, S, kts, w, s);
         return (a.K % GK == 0) ? launch_tile<T, BM, BN, P, true>(a, S, kts, w, s) : launch_tile<T, BM, BN, P, false>(a, S, kts, w, s);
     }
 }
 
-struct Plan { int idx, S, kts; };
+// full >= 0: 256 x 192 tiles, the first `full` whole and each of the rest in S pieces of kts K steps (S > 1)
+struct Plan { int idx, S, kts, full = -1; };
 
 
 // blocks of one tile shape resident per CU (LDS and registers), queried once per process
@@ -941,7 +991,7 @@ template <int T>
 struct Cand {
     int bm, bn;
     int (*occ)();
-    int (*launch)(const Args&, int, int, const Workspace&, hipStream_t);
+    int (*launch)(const Args&, int, int, int, const Workspace&, hipStream_t);
 };
 
 template <int T, int BM, int BN, int P>
@@ -953,6 +1003,7 @@ static const Cand<T> CANDS[] = {cand<T, 256, 256, 1>(), cand<T, 256, 192, 1>(), 
                                 cand<T, 128, 64, 3>(),  cand<T, 64, 256, 3>(),  cand<T, 64, 192, 3>(),
                                 cand<T, 64, 128, 3>(),  cand<T, 64, 64, 3>()};
 
+constexpr int SG_IDX = 1;                        // the 256 x 192 tile's place in CANDS
 // K-step time (us) of one block of each candidate when it runs alone on its CU (the order of CANDS; 256 x 192 without a
 // split is the specialized-wave kernel)
 static constexpr double T1_US[] = {1.56, 1.20, 1.14, 1.10, 1.04, 0.83, 0.57, 0.84, 0.80, 0.58, 0.43};
@@ -965,6 +1016,16 @@ static constexpr double T1_US[] = {1.56, 1.20, 1.14, 1.10, 1.04, 0.83, 0.57, 0.8
 // 27B-class layer. Its choices run within 5 % of the fastest candidate on 38 of those 40 shapes (all 40 together 0.3 %
 // over the fastest), where the model below (fitted to loaded CUs of one tile shape) lost 15 % (512 rows: 1.6-1.9x).
 constexpr double PG_G2 = 1.44, PG_G3 = 2.11, PG_SGX = 1.18, PG_SA = 8.4, PG_SB = 22.5;
+// Pieces: 256 x 192 tiles on the specialized kernel, whole in whole rounds of the CUs, the tiles of the last, partial round
+// cut along K into S pieces (a 512 x 34816 x 5120 product is 364 tiles: 256 whole, 108 in two pieces each, 1.5 rounds for 2).
+// A K step takes PP_T us, PP_L more as the busy CUs rise from PP_B to all of them (the clock falls); the pieces add PP_A us
+// (fill, and the kernel that sums them) and PP_W us per MB of partials. Fitted, as is PP_C, to 208 shapes of Q4_K tiles and
+// 43 of int8 and Q6_K (65-2048 rows, 13 weights of 1024 to 34816 rows), every plan timed: where the pieces' time is below
+// PP_C of the model's best they ran faster on 62 of the 63 shapes they were chosen for, by up to 28 % (Q4_K 256 x 5120 x
+// 17408 79 -> 55 us, 512 x 34816 x 5120 185 -> 167, 512 x 5120 x 17408 106 -> 93), and 5 % slower on one.
+constexpr double PP_T = 0.92, PP_L = 0.33, PP_B = 108, PP_A = 12, PP_W = 0.15, PP_C = 0.93;
+// At least 12 K steps a piece (11: 768 x 2816 x 2816 30.5 -> 31.2 us).
+constexpr int PP_MAX = 12, PP_MIN = 12;
 
 template <int T>
 static Plan plan_wide(int64_t M, int64_t N, int64_t K, int cus) {
@@ -989,6 +1050,16 @@ static Plan plan_wide(int64_t M, int64_t N, int64_t K, int cus) {
             if (S > 1) t += PG_SA + PG_SB * (double)(S * bm * bn * 4) / 1e6;
             if (t < best_t) best_t = t, best = Plan{i, (int)S, (int)kts};
         }
+    }
+    const int64_t tiles = sg_tiles(M, N), whole = tiles / cus * cus, rest = tiles - whole;
+    auto step = [&](int64_t blocks) { return PP_T * (1.0 + PP_L * std::max(0.0, ((double)blocks - PP_B) / ((double)cus - PP_B))); };
+    best_t *= PP_C;
+    for (int64_t S0 = 2; S0 <= PP_MAX && M > SG_BM / 2 && rest > 0 && cus > PP_B; ++S0) {
+        const int64_t kts = (KT + S0 - 1) / S0, S = (KT + kts - 1) / kts, blocks = rest * S, bytes = blocks * SG_BM * SG_BN * 4;
+        if (S != S0 || kts < PP_MIN || rest > SCRATCH_TILES || (size_t)bytes > std::min(WS_BYTES, SCRATCH_BYTES)) continue;
+        const double t = (double)(whole / cus * KT) * step(cus) + (double)kts * ((double)(blocks / cus) * step(cus) + (blocks % cus ? step(blocks % cus) : 0.0)) +
+                         PP_A + PP_W * (double)bytes / 1e6;
+        if (t < best_t) best_t = t, best = Plan{SG_IDX, (int)S, (int)kts, (int)whole};
     }
     return best;
 }
@@ -1121,11 +1192,18 @@ static int launch_gemm_t(const Args& a, hipStream_t s) {
     Plan p;
     if (int rc = pick<T>(a, &p)) return rc;
     Workspace w;
-    if (p.S > 1) {
+    if (p.full >= 0) {
+        // without a workspace (a first call under capture, more streams than sets) the pieces' tiles run whole
+        const int64_t rest = sg_tiles(a.M, a.N) - p.full;
+        if (split_workspace(a, rest, (size_t)rest * p.S * SG_BM * SG_BN * 4, s, &w) != 0) {
+            set_error(0, "");
+            p.S = 1;
+        }
+    } else if (p.S > 1) {
         const int64_t tiles = ((a.M + CANDS<T>[p.idx].bm - 1) / CANDS<T>[p.idx].bm) * ((a.N + CANDS<T>[p.idx].bn - 1) / CANDS<T>[p.idx].bn);
         if (int rc = split_workspace(a, tiles, (size_t)tiles * p.S * CANDS<T>[p.idx].bm * CANDS<T>[p.idx].bn * 4, s, &w)) return rc;
     }
-    return CANDS<T>[p.idx].launch(a, p.S, p.kts, w, s);
+    return CANDS<T>[p.idx].launch(a, p.S, p.kts, p.full, w, s);
 }
 
 int gemm_plan(int t, const Args& a, int* kernel, int* bm, int* bn, int* splits) {
