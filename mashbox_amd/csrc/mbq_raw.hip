@@ -69,7 +69,10 @@ __global__ __launch_bounds__(64 * RV_W) void raw_gemv_kernel(const uint8_t* __re
             else raw_load<T>(fl.u, row, u < U ? u : U - 1);
         };
         load(ks);
-        if (c0) __syncthreads();                                         // the last chunk's x has been read
+        if (c0) {                                                        // the last chunk's x has been read
+            wait_lgkm0();                                                // (and no LDS write of the wave is in flight)
+            __syncthreads();
+        }
         for (int q = threadIdx.x; q < M * (kc >> 3); q += 64 * RV_W) {
             const int m = q / (kc >> 3), p = q % (kc >> 3);              // piece p: unit p / 4, its piece p % 4
             st16(xs + m * KC + (p >> 5) * 256 + ((p & 3) * 8 + ((p >> 2) & 7)) * 8, ld16(x + (int64_t)m * K + c0 + 8 * p));
