@@ -22,11 +22,31 @@ static int check_launch(const char* what) {
     return 0;
 }
 
+// 8 values -> NT bfloat16 operands whose sum they are
+template <int NT>
+__device__ __forceinline__ void raw_split(const float v[8], bf16x8_t b[NT]) {
+#pragma clang fp contract(off)                                          // v's own bits: not the product behind them, unrounded
+    uint32_t t[NT][4];
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = v[e];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) t[k][e >> 1] = __builtin_amdgcn_perm(__float_as_uint(f[e + 1]), __float_as_uint(f[e]), 0x07060302u);
+        if (k + 1 < NT)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] -= __uint_as_float(__float_as_uint(f[e]) & 0xFFFF0000u);
+        b[k] = __builtin_bit_cast(bf16x8_t, u32x4{t[k][0], t[k][1], t[k][2], t[k][3]});
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ 1-8 rows
 // Each lane takes one 32-value unit at a time and multiplies it with up to MR activation rows: the types of codes
 // (raw_coded) as bfloat16 pairs with v_dot2_f32_bf16, float32 sums of exact products that the scale multiplies once (a unit
-// that meets a scale, an activation or a sum that is not finite: value by value); the others (F16, F32, TQ1_0) value by
-// value with float32 FMAs, a unit's sum added to the row's. Bound: the vector work (2.5 to 4 instructions per value at one row) and, below about 20 MB, the
+// that meets a scale, an activation or a sum that is not finite: value by value); F16 at 5-8 rows as two
+// bfloat16 terms per value (1024 x 5120 at 8 rows 13.5 us value by value, 10.9 so); F32, TQ1_0 and F16 at 1-4 rows value by
+// value with float32 FMAs (F16 34816 x 5120 at 4 rows 68 us, 77 as two terms). A unit's sum is added to the row's. Bound: the vector work (2.5 to 4 instructions per value at one row) and, below about 20 MB, the
 // launch's fill and drain. Against a float64 product it is off by 0.6e-7 to 1.5e-7 (one to eight rows, K 512 to 17408).
 //
 // 8 lanes take 8 consecutive units of a weight row (a super-block of the 256-value types: lane j always its sub-block j, so
@@ -39,7 +59,7 @@ static int check_launch(const char* what) {
 // 5120 x 17408 56 -> 17, 8192 x 5120 24 -> 9.6; IQ4_XS 112 -> 29, 60 -> 18; Q5_0 59 -> 35, 28 -> 21; F16 63 -> 60. Four
 // rows: Q3_K 34816 x 5120 128 -> 43. Two rows of weights per lane (half the LDS reads of x) ran 2 % faster on 34816 rows and
 // 10-20 % slower below 8192, 4 waves per block 5-15 % slower at 5120 x 17408: neither is kept.
-constexpr int RV_W = 8, RV_X1 = 40 * 1024, RV_X = 64 * 1024;
+constexpr int RV_W = 8, RV_X1 = 40 * 1024, RV_X = 64 * 1024, RV_XL = 128 * 1024;
 
 // a step's bytes in flight: a 16-byte piece of a super-block (raw_shared), else the unit itself
 template <int T, bool SH = raw_shared<T>()> struct RawFlight { RawRegs<T> u; };
@@ -125,10 +145,30 @@ __global__ __launch_bounds__(64 * RV_W) void raw_gemv_kernel(const uint8_t* __re
                         if constexpr (raw_min<T>()) d[m] = __builtin_fmaf(sc.b[h], sx[m], d[m]);
                     }
                 }
+                done = raw_finite<T>(sc);
+            } else if constexpr (T == T_F16 && MR == 8) {                // two exact terms: a dot2 each for two values
+                done = true;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    float v[8];
+                    bf16x8_t b[2];
+                    raw_vals<T>(cur, sc, u, s, v);
+                    raw_split<2>(v, b);
+                    const u32x4 hi = __builtin_bit_cast(u32x4, b[0]), lo = __builtin_bit_cast(u32x4, b[1]);
+#pragma unroll
+                    for (int m = 0; m < MR; ++m) {
+                        if (m >= M) break;
+                        const u32x4 q = ld16(xp + m * KC + s * 64);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) d[m] = dot2(lo[e], q[e], dot2(hi[e], q[e], d[m]));
+                    }
+                }
+            }
+            if (done) {
                 float f = 0.f;                                           // a non-finite scale, activation or sum makes it NaN
 #pragma unroll
                 for (int m = 0; m < MR; ++m) f = __builtin_fmaf(0.f, d[m], f);
-                done = f == 0.f && raw_finite<T>(sc);
+                done = f == 0.f;
             }
             if (!done) {
 #pragma unroll
@@ -176,13 +216,14 @@ template <int T, int MR>
 static int raw_gemv_m(const uint8_t* raw, const uint16_t* x, int64_t M, int64_t N, int64_t K, void* y, int out_bf16, hipStream_t s) {
     int KS = N < 8192 ? 8 : 4;
     while (KS > 1 && KS * 256 > K) KS /= 2;
-    const int64_t KC = std::min<int64_t>((K + 255) / 256 * 256, (M == 1 ? RV_X1 : RV_X) / (2 * M) / 256 * 256);
+    const int64_t rows = RV_W / KS * 8, blocks = (N + rows - 1) / rows;
+    const int64_t X = M == 1 ? RV_X1 : blocks <= cus_of_device() ? RV_XL : RV_X;
+    const int64_t KC = std::min<int64_t>((K + 255) / 256 * 256, X / (2 * M) / 256 * 256);
     const size_t lds = (size_t)(M * KC) * 2 + (size_t)RV_W * 8 * (MR * 4 + (raw_shared<T>() ? RAW_SLOT : 0));
     auto kern = raw_gemv_kernel<T, MR>;
     static std::atomic<uint64_t> set{0};
-    if (set_lds_limit((const void*)kern, 80 * 1024, set) != hipSuccess) return set_error(MBQ_LAUNCH_FAIL, "raw GEMV: %zu bytes of LDS refused", lds);
-    const int64_t rows = RV_W / KS * 8;
-    kern<<<dim3((unsigned)((N + rows - 1) / rows)), 64 * RV_W, lds, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16, KS, (int)KC);
+    if (set_lds_limit((const void*)kern, RV_XL + 16 * 1024, set) != hipSuccess) return set_error(MBQ_LAUNCH_FAIL, "raw GEMV: %zu bytes of LDS refused", lds);
+    kern<<<dim3((unsigned)blocks), 64 * RV_W, lds, s>>>(raw, x, (int)M, (int)N, (int)K, y, out_bf16, KS, (int)KC);
     return check_launch("raw GEMV");
 }
 
@@ -263,25 +304,6 @@ __device__ __forceinline__ float raw_dot(const uint8_t* row, const uint16_t* x, 
 
 // element offset of chunk c (8 values) of row r in an x stage
 __device__ __forceinline__ int rg_off(int r, int c) { return r * RG_K + ((c ^ ((r >> 1) & 7)) << 3); }
-
-// 8 values -> NT bfloat16 operands whose sum they are
-template <int NT>
-__device__ __forceinline__ void raw_split(const float v[8], bf16x8_t b[NT]) {
-#pragma clang fp contract(off)                                          // v's own bits: not the product behind them, unrounded
-    uint32_t t[NT][4];
-    float f[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = v[e];
-#pragma unroll
-    for (int k = 0; k < NT; ++k) {
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) t[k][e >> 1] = __builtin_amdgcn_perm(__float_as_uint(f[e + 1]), __float_as_uint(f[e]), 0x07060302u);
-        if (k + 1 < NT)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] -= __uint_as_float(__float_as_uint(f[e]) & 0xFFFF0000u);
-        b[k] = __builtin_bit_cast(bf16x8_t, u32x4{t[k][0], t[k][1], t[k][2], t[k][3]});
-    }
-}
 
 // Types whose 32 values share one scale and whose codes need no more than a bfloat16's 8 bits (raw_factored): one MFMA per
 // code instead of three per value. Both lane halves hold the same unit (half h its values 8h .. + 7 and 16 + 8h .. + 7, the
