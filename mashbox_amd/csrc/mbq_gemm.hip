@@ -802,20 +802,29 @@ __global__ __launch_bounds__(256) void sgemm_sum_kernel(const GemmArgs g) {
 // split-K call yet on the device, or the spare taken by another capturing stream since the last eager call) is refused
 // with an error and launches nothing. Graphs recorded on one stream share its set: replays of two such graphs must not
 // overlap in time. A destroyed stream's set is kept (a later stream at the same handle reuses it).
-constexpr int WS_MAX_STREAMS = 32;            // sets per device (each WS_BYTES + WS_TILES counters), spare included
+//
+// A call that can do without (the pieces of the specialized kernel, whose tiles can also run whole) takes a set that its
+// stream holds, or one of as many sets again with a spare of their own, so that it leaves no split-K call without one; a
+// failed allocation of these is not tried again.
+constexpr int WS_MAX_STREAMS = 32;            // sets per device and kind (each WS_BYTES + WS_TILES counters), spare included
 
 static int ws_alloc(Workspace* w, int dev) {
     // Uncached device memory: no L2 holds its lines, so a partial one XCD stores is what another XCD loads after the
     // arrival count, with no cache write-back or invalidation between (the exchange of every split-K kernel). Never
-    // freed, also on a failed set-up.
+    // freed once a kernel may have used it. A failure here is not left for the launch check of a call that goes on.
     void *p = nullptr, *c = nullptr;
-    if (hipExtMallocWithFlags(&p, WS_BYTES, hipDeviceMallocUncached) != hipSuccess)
+    if (hipExtMallocWithFlags(&p, WS_BYTES, hipDeviceMallocUncached) != hipSuccess) {
+        (void)hipGetLastError();
         return set_error(MBQ_LAUNCH_FAIL, "GEMM: split-K workspace allocation on device %d failed", dev);
+    }
     // the counters are zeroed on the null stream and waited for here, once: the first kernel that uses them may run on
     // a non-blocking stream, which does not wait for the null stream
-    if (hipExtMallocWithFlags(&c, WS_TILES * sizeof(int), hipDeviceMallocUncached) != hipSuccess ||
-        hipMemset(c, 0, WS_TILES * sizeof(int)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+    const bool have = hipExtMallocWithFlags(&c, WS_TILES * sizeof(int), hipDeviceMallocUncached) == hipSuccess;
+    if (!have || hipMemset(c, 0, WS_TILES * sizeof(int)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
+        if (!have) (void)hipFree(p);                                      // nothing has touched it
+        (void)hipGetLastError();
         return set_error(MBQ_LAUNCH_FAIL, "GEMM: split-K counter allocation on device %d failed", dev);
+    }
     w->ws = static_cast<float*>(p);
     w->cnt = static_cast<int*>(c);
     w->bytes = WS_BYTES;
@@ -824,42 +833,51 @@ static int ws_alloc(Workspace* w, int dev) {
     return 0;
 }
 
-int workspace(Workspace* out, hipStream_t s) {
-    struct Dev { hipStream_t stream[WS_MAX_STREAMS]; Workspace set[WS_MAX_STREAMS]; int n = 0; Workspace spare; };
+static int workspace(Workspace* out, hipStream_t s, bool optional) {
+    struct Kind { int n = 0; Workspace spare; bool failed = false; };     // split-K calls' sets; those of calls that can do without
+    struct Dev { hipStream_t stream[2 * WS_MAX_STREAMS]; Workspace set[2 * WS_MAX_STREAMS]; int n = 0; Kind kind[2]; };
     static Dev per_dev[64];
     static std::mutex mu;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return set_error(MBQ_LAUNCH_FAIL, "GEMM: no device");
     std::lock_guard<std::mutex> lk(mu);
     Dev& d = per_dev[dev];
+    Kind& k = d.kind[optional];
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     const bool capturing = hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
-    // sets held: d.n streams' and the spare, at most WS_MAX_STREAMS; the spare is refilled by eager calls (best effort:
-    // a failed refill only means that a later first capture on a new stream is refused)
-    auto refill = [&] { if (!capturing && !d.spare.ws && d.n < WS_MAX_STREAMS) ws_alloc(&d.spare, dev); };
+    // sets held of a kind: k.n streams' and the spare, at most WS_MAX_STREAMS; the spare is refilled by eager calls (best
+    // effort: a failed refill only means that a later first capture on a new stream is refused)
+    auto refill = [&] {
+        if (!capturing && !k.failed && !k.spare.ws && k.n < WS_MAX_STREAMS && ws_alloc(&k.spare, dev) != 0) k.failed = optional;
+    };
     for (int i = 0; i < d.n; ++i)
         if (d.stream[i] == s) {
             *out = d.set[i];
             refill();
             return 0;
         }
-    if (!capturing && d.n + (d.spare.ws ? 1 : 0) >= WS_MAX_STREAMS)
+    if (!capturing && k.n + (k.spare.ws ? 1 : 0) >= WS_MAX_STREAMS)
         return set_error(MBQ_BAD_ARG, "GEMM: split-K calls on more than %d streams of device %d (one workspace each)",
                          WS_MAX_STREAMS - 1, dev);
     Workspace w;
     if (capturing) {
-        if (!d.spare.ws)
+        if (!k.spare.ws)
             return set_error(MBQ_BAD_ARG, "GEMM: the first split-K call on this stream of device %d needs a workspace, "
                                           "which a stream being captured into a graph cannot allocate: make one eager "
                                           "call first", dev);
-        w = d.spare;
-        d.spare = Workspace{};
+        w = k.spare;
+        k.spare = Workspace{};
     } else {
-        if (int rc = ws_alloc(&w, dev)) return rc;
+        if (k.failed) return set_error(MBQ_LAUNCH_FAIL, "GEMM: no workspace on device %d", dev);
+        if (int rc = ws_alloc(&w, dev)) {
+            k.failed = optional;
+            return rc;
+        }
     }
     d.stream[d.n] = s;
     d.set[d.n] = w;
     ++d.n;
+    ++k.n;
     refill();
     *out = w;
     return 0;
@@ -900,13 +918,13 @@ static int scratch_workspace(hipStream_t s, Workspace* out) {
     return 0;
 }
 
-int split_workspace(const Args& a, int64_t tiles, size_t bytes, hipStream_t s, Workspace* out) {
+int split_workspace(const Args& a, int64_t tiles, size_t bytes, hipStream_t s, Workspace* out, bool optional) {
     const size_t cap = a.noalloc ? SCRATCH_BYTES : WS_BYTES;
     const int ntiles = a.noalloc ? SCRATCH_TILES : WS_TILES;
     if (tiles > ntiles || bytes > cap)                                // checked before any set-up: nothing launches
         return set_error(MBQ_BAD_ARG, "GEMM: a split-K plan of %lld tiles and %zu partial bytes exceeds the %s (%d tiles, %zu bytes)",
                          (long long)tiles, bytes, a.noalloc ? "scratch of mbq_matmul_noalloc" : "workspace", ntiles, cap);
-    return a.noalloc ? scratch_workspace(s, out) : workspace(out, s);
+    return a.noalloc ? scratch_workspace(s, out) : workspace(out, s, optional);
 }
 
 // ------------------------------------------------------------------------------------------------- launchers
@@ -1195,7 +1213,7 @@ static int launch_gemm_t(const Args& a, hipStream_t s) {
     if (p.full >= 0) {
         // without a workspace (a first call under capture, more streams than sets) the pieces' tiles run whole
         const int64_t rest = sg_tiles(a.M, a.N) - p.full;
-        if (split_workspace(a, rest, (size_t)rest * p.S * SG_BM * SG_BN * 4, s, &w) != 0) {
+        if (split_workspace(a, rest, (size_t)rest * p.S * SG_BM * SG_BN * 4, s, &w, true) != 0) {
             set_error(0, "");
             p.S = 1;
         }

@@ -40,11 +40,11 @@ constexpr int SCRATCH_TILES = 4096;
 // partials through it release and acquire at agent scope (split_release / split_acquire); the allocated workspace is
 // uncached device memory, which no L2 holds, so its device-coherent stores and loads need no fence
 struct Workspace { float* ws = nullptr; int* cnt = nullptr; size_t bytes = 0; int tiles = 0; int fenced = 0; };
-int workspace(Workspace* out, hipStream_t s);   // refused while s is capturing and nothing is allocated yet
 // The workspace of a split-K launch whose partial tiles take `bytes` over `tiles` arrival counters: the static scratch
 // array when a.noalloc (mbq_matmul_noalloc; never allocated), else the allocated per-device workspace. An error, with
-// nothing launched, when the plan does not fit it.
-int split_workspace(const Args& a, int64_t tiles, size_t bytes, hipStream_t s, Workspace* out);
+// nothing launched, when the plan does not fit it, or when s is capturing and no set is allocated for it. optional: the
+// caller can do without, and leaves the sets and the spare of the calls that cannot as they are.
+int split_workspace(const Args& a, int64_t tiles, size_t bytes, hipStream_t s, Workspace* out, bool optional = false);
 
 // largest weight plane or activation range a kernel addresses through a buffer resource (32-bit offsets; below the
 // out-of-range offset OOB_VOFF of mbq_device.h)

@@ -127,3 +127,47 @@ def test_recorded_before_and_after_an_eager_call():
     sys.stdout.write(r.stdout)
     sys.stderr.write(r.stderr[-4000:])
     assert r.returncode == 0 and "pieces capture ok" in r.stdout
+
+
+SPARE_SCRIPT = r"""
+import sys
+sys.path.insert(0, sys.argv[1])
+import torch
+import tests.test_gpu_gemm_pieces as P
+from mashbox_amd import _lib as LIB
+dev = torch.device("cuda", 0)
+L = LIB.lib()
+a, b = (512, 5120, 6144), (16, 1024, 5120)                  # pieces; a K split that has no other form
+ta, bufa, wa = P._weight(12, *a[1:], dev)
+pb = P.KQ.repack_host(12, P.G.RAW[12](P.np.random.default_rng(4), *b[1:]), b[1:]).to(dev)
+tb, bufb = pb.t, pb.buf
+assert LIB.gemm_plan(tb, *b)[3] > 1, "the case must split K"
+xa, xb = P._x(a[0], a[2], dev), P._x(b[0], b[2], dev)
+ya, yb = torch.empty(a[:2], device=dev), torch.empty(b[:2], device=dev)
+eager = P._call(L.mbq_matmul, tb, bufb, xb, *b, torch.empty_like(yb))
+torch.cuda.synchronize()
+ga, gb = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+with torch.cuda.graph(ga, stream=torch.cuda.Stream()):
+    P._call(L.mbq_matmul, ta, bufa, xa, *a, ya)
+with torch.cuda.graph(gb, stream=torch.cuda.Stream()):
+    P._call(L.mbq_matmul, tb, bufb, xb, *b, yb)
+for _ in range(3):
+    ya.zero_(), yb.zero_()
+    ga.replay()
+    gb.replay()
+    torch.cuda.synchronize()
+    P.assert_product_dev(ya, xa.double() @ wa.T, "pieces' product")
+    assert torch.equal(yb, eager)
+    P._call(L.mbq_matmul, tb, bufb, xb, *b, torch.empty_like(yb))
+print("spare ok", flush=True)
+"""
+
+
+@pytest.mark.gpu
+def test_pieces_leave_the_spare_workspace_to_split_k():
+    """after one eager split-K call, a pieces product recorded on one new stream and a split-K product on another: the first
+    can do without a workspace, the second is refused without one"""
+    r = subprocess.run([sys.executable, "-c", SPARE_SCRIPT, ROOT], capture_output=True, text=True, timeout=110)
+    sys.stdout.write(r.stdout)
+    sys.stderr.write(r.stderr[-4000:])
+    assert r.returncode == 0 and "spare ok" in r.stdout
