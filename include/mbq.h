@@ -138,7 +138,7 @@ int mbq_matmul(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* l
  * library runs on holds its own copy until the process ends), instead of mbq_matmul's allocated workspace. A plan whose
  * partials exceed the scratch (none of the automatic plans on up to 256 CUs; a forced plan can) returns MBQ_E_ARG and
  * launches nothing. Every call on one GPU shares that GPU's scratch: calls that overlap in time on one GPU (two streams)
- * race, and must not both split K. */
+ * race, and must not both split K (mbq_gemm_plan says which do: splits > 1, the 256 x 192 tiles' K pieces among them). */
 int mbq_matmul_noalloc(int t, const uint8_t* planes_dev, int64_t layer, const int32_t* layer_dev, int64_t nlayers,
                        const uint16_t* x_dev, int64_t M, int64_t N, int64_t K, void* y_dev, int out_dtype, void* stream);
 
@@ -181,7 +181,7 @@ int mbq_matmul_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t
 /* The same product for any number of activation rows (M >= 1), on the bfloat16 matrix cores with float32 accumulation:
  * each weight value, bit for bit mbq_dequant_raw's, is cut into one to three bfloat16 terms whose sum it is exactly, so
  * every product is exact as the float32 product of a bfloat16 x is up to its own rounding. Types, shapes and alignments
- * as mbq_matmul_raw. work_dev: at least mbq_gemm_raw_work(M, N, K) bytes of device memory (16-byte aligned; NULL when
+ * as mbq_matmul_raw, and 256 rows of x (or all M) within 2 GiB. work_dev: at least mbq_gemm_raw_work(M, N, K) bytes of device memory (16-byte aligned; NULL when
  * that is 0) for the float32 partials of the K ranges, free again when the call's work on the stream is done. */
 int mbq_gemm_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M, int64_t N, int64_t K, void* y_dev,
                  int out_dtype, void* work_dev, int64_t work_bytes, void* stream);

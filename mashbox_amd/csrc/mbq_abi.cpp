@@ -330,6 +330,8 @@ int mbq_gemm_raw(int t, const uint8_t* raw_dev, const uint16_t* x_dev, int64_t M
     if (M == 0) return MBQ_OK;
     if (M < 0 || M > INT32_MAX) return set_error(MBQ_BAD_ARG, "gemm_raw: M = %lld", (long long)M);
     if (int rc = raw_product_args("gemm_raw", t, raw_dev, x_dev, M, N, K, y_dev)) return rc;
+    if (std::min<int64_t>(M, 256) * K > 0x3FFFFFFF)                        // a tile's rows of x are one buffer range
+        return set_error(MBQ_BAD_ARG, "gemm_raw: 256 rows of x take more than 2 GiB (K = %lld)", (long long)K);
     const int64_t need = raw_gemm_work(M, N, K);
     if (work_bytes < need || (need > 0 && (!work_dev || !aligned16(work_dev))))
         return set_error(MBQ_BAD_ARG, "gemm_raw: %lld bytes of work needed (16-byte aligned), %lld given", (long long)need, (long long)work_bytes);

@@ -455,7 +455,7 @@ def _raw_product(x: torch.Tensor, h: "Raw") -> torch.Tensor | None:
     rows, cols = h.shape[-2:]
     m = x.shape[:-1].numel()
     if (x.dtype != torch.bfloat16 or m < 1 or h.t in (2, 8, 12, 13, 14) or cols % max(32, TYPES[h.t][1])
-            or (m > RAW_GEMV_MAX_M and (max(m * cols, m * rows) > 0x7FFFFFFF or not _untraced(x)))):
+            or (m > RAW_GEMV_MAX_M and (max(m * cols, m * rows, 2 * min(m, 256) * cols) > 0x7FFFFFFF or not _untraced(x)))):
         return None                                  # (the kernel types' blocks, off the kernels: rebuild and GEMM)
     raw = h.raw
     if raw.dim() != 2 or not raw.is_contiguous() or raw.shape[0] != rows or raw.shape[1] != row_bytes(h.t, cols):
